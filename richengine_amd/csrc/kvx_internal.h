@@ -140,6 +140,27 @@ inline uint32_t verify_block_rows(uint32_t format, uint32_t fused_rows) {
   if (format == KVX_FMT_INT4 && 26 * by48 < 15 * by32) return 48;
   return 32;
 }
+// Whether a chunk runs as workgroups of 256 fused rows that share their pages (kvx_prefill.hip)
+// rather than as waves and workgroups of single tiles, which spread a small call over more
+// CUs.  A function of the sequence alone: a batch gives a sequence the bits of its own call.
+// Times are one layer's call, tiles / workgroups of 256:
+//  head dimension 256: bf16, int8 and e4m3 pages in one split always (64 rows after 32 tokens, bf16
+//    32.3 / 17.7 us; 8 rows even or better), under several from 64 rows (64 rows after 512 tokens, fp8
+//    40.1 / 35.2) or 20 000 fused rows of work items on (33 rows over 8192 tokens in 28 splits, bf16
+//    61 / 38; in 2 splits 20.6 / 29.1).  int4 pages under several splits from 40 000 on (over 8192
+//    tokens in 5 splits: 256 rows, 30 720, 117 / 127 us; 512 rows 162 / 140).
+//  64 and 128: from 32 768 and 40 000 on (64 rows over 8192 tokens in 32 splits: 64-wide bf16, 65 536,
+//    33 / 28 us, 128-wide 32 768, 29 / 34; 128 rows 40.4 / 37.8), where the splits hold more than a
+//    page: below, sharing has nothing to share.
+inline bool prefill_by_chunk(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
+  const uint32_t D = l.head_dim, H = l.kv_heads, G = query_heads / H;
+  const uint64_t work = uint64_t(p.rows) * G * H * p.split_count;
+  if (D == 256 && l.format == KVX_FMT_INT4) return p.split_count > 1 && work >= 40000;
+  if (D == 256) return p.split_count == 1 || p.rows >= 64 || work >= 20000;
+  if (D != 64 && D != 128) return false;
+  const uint64_t pages = (uint64_t(p.committed_tokens) + p.rows + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS;
+  return pages > p.split_count && work >= (D == 64 ? 32768u : 40000u);
+}
 // Whether tiles 2i and 2i + 1 of a chunked prefill that starts after `committed`
 // tokens see the same number of pages, for every i: tile 2i sees committed + 16 i
 // + 8 tokens, its neighbour 8 more, and no page boundary lies in between exactly
@@ -167,12 +188,9 @@ inline bool prefill_pairs_with_splits(uint32_t format, uint32_t committed, uint3
   if (format == KVX_FMT_INT4 && tiles < 64) return false;
   return 2ull * prefill_paired_waves(tiles, kv_heads, group) * splits >= prefill_paired_slots(format);
 }
-// bf16, fp8 and int8 pages of head dimension 256: chunks from kGroupedPrefillRows rows on run
-// in lanes of four (or two) tiles, for a workgroup of four waves that fetches every page
-// once for all of them and shares it through LDS, where the lane's fused rows fit three
-// blocks of 16 per wave (192).  Measured from 64-row chunks up (two lanes per KV head, under
-// the plan's 32 splits): 0.085 against 0.12 ms on bf16 pages after 16 K tokens.
-// 0 = no such lanes for this shape.
+// What kvx_prefill_plan counts on bf16, fp8 and int8 pages of head dimension 256: chunks from
+// kGroupedPrefillRows rows on as groups of four (or two) tiles, up to 192 fused rows, that share
+// a workgroup and its pages.  0 = no such groups for this shape.
 constexpr uint32_t kGroupedPrefillRows = 64;
 inline uint32_t prefill_group_width(uint32_t format, uint32_t head_dim, uint32_t rows, uint32_t group) {
   if (format == KVX_FMT_INT4 || head_dim != 256 || rows < kGroupedPrefillRows) return 0;
@@ -181,9 +199,8 @@ inline uint32_t prefill_group_width(uint32_t format, uint32_t head_dim, uint32_t
   // Groups of one or two query heads would leave three quarters of every wave's rows empty.
   return width * tile_fused >= 96 ? width : 0u;
 }
-// Whether the tiles of every such lane see the same number of pages, so that a lane cut into
-// splits is each of its tiles cut into splits: lanes of four tiles (32 rows) when the chunk
-// starts on a page boundary, lanes of two as for pairs.
+// Whether the tiles of every such group see the same number of pages: groups of four tiles
+// (32 rows) when the chunk starts on a page boundary, groups of two as for pairs.
 inline bool prefill_group_splits_alike(uint32_t width, uint32_t committed) {
   return width == 4 ? committed % KVX_PAGE_TOKENS == 0 : prefill_tiles_pair(committed);
 }

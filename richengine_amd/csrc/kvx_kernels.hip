@@ -1804,6 +1804,11 @@ int kvx_attend_wide_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t
                            hipStream_t stream, Tiles tile_rows = 0,
                            const Epilogue *epilogue = nullptr);
 
+int kvx_prefill_chunk_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t query_heads,
+                             const void *queries, void *output, const uint64_t *const *page_tables,
+                             const kvx_prefill_params *params, uint32_t sequences,
+                             uint64_t sequence_stride, void *workspace, hipStream_t stream);
+
 // int4 pages go to their own kernels, bf16, fp8 and int8 pages to the wide-element
 // ones; 1 = neither covers the shape.
 static int attend_matrix(const kvx_storage *s, kvx_kv_layer kv, uint32_t query_heads,
@@ -2558,7 +2563,7 @@ int kv_append_attend_decode_hidden(const kvx_storage *s, uint32_t layer, const v
 }
 
 namespace {
-// How the tiles of a chunk go to the matrix-core kernels.
+// How the tiles of a chunk that stays tile by tile (prefill_by_chunk) go to the matrix-core kernels.
 // With a single split every tile walks its pages from the first, so two
 // neighbouring tiles can share one walk as a lane of 16 rows: a row's softmax
 // runs over the same pages in the same order (the page the second tile may
@@ -2568,9 +2573,6 @@ namespace {
 // splits, which they do when they see the same number of pages
 // (prefill_tiles_pair: true for every pair of the chunk, or for none), and pay
 // only where the paired launch fills the GPU (prefill_pairs_with_splits).
-// bf16, fp8 and int8 pages: lanes of four (or two) tiles for a workgroup that shares
-// every page through LDS (prefill_group_width); with several splits only where a
-// lane's tiles cut their pages alike.
 struct TileShape {
   uint32_t width;  // tiles per lane
   int lane_kind;   // attend_matrix's many_tiles
@@ -2694,6 +2696,12 @@ int kv_attend_prefill(const kvx_storage *s, uint32_t layer, uint32_t query_heads
   if (workspace_bytes < partial_bytes + rows * 2 * sizeof(float))
     return fail(KVX_EINVAL, "prefill attention scratch is smaller than its bound");
   auto st = static_cast<hipStream_t>(stream);
+  if (kvx::prefill_by_chunk(l, query_heads, *params)) {
+    const int fast = kvx_prefill_chunk_launch(s, kv, query_heads, queries, output, &page_table, params, 1, 0,
+                                              workspace, st);
+    if (D == 256) took(fast);
+    if (fast <= 0) return fast;
+  }
   {
     const int fast = prefill_matrix(s, kv, query_heads, queries, output, &page_table, params, 1, 0,
                                     workspace, workspace_bytes, st);
@@ -2767,7 +2775,8 @@ int kv_attend_prefill_batch(const kvx_storage *s, uint32_t layer, uint32_t query
   // Nothing is enqueued unless every sequence is valid.
   const uint32_t G = query_heads / l.kv_heads;
   uint64_t rows = 0;
-  bool alike = true;
+  bool alike = true, same = true;
+  uint32_t by_chunk = 0;
   for (uint32_t q = 0; q < n_sequences; ++q) {
     if (!page_tables[q]) return fail(KVX_EINVAL, "null page table");
     if (int rc = validate_prefill(l, query_heads, params[q])) return rc;
@@ -2775,9 +2784,11 @@ int kv_attend_prefill_batch(const kvx_storage *s, uint32_t layer, uint32_t query
         sequence_stride < uint64_t(l.kv_heads) * params[q].chunk_stride * G * l.head_dim)
       return fail(KVX_EINVAL, "sequence stride is smaller than a sequence's chunk");
     rows += prefill_rows(l, query_heads, params[q]);
-    alike = alike && params[q].rows == params[0].rows &&
-            params[q].chunk_stride == params[0].chunk_stride &&
-            params[q].split_count == params[0].split_count &&
+    same = same && params[q].rows == params[0].rows &&
+           params[q].chunk_stride == params[0].chunk_stride &&
+           params[q].split_count == params[0].split_count;
+    by_chunk += kvx::prefill_by_chunk(l, query_heads, params[q]) ? 1u : 0u;
+    alike = alike && same && !by_chunk &&
             tile_shape(l, query_heads, params[q]) == tile_shape(l, query_heads, params[0]);
   }
   if (workspace_bytes < rows * l.head_dim * sizeof(float) + 256 + rows * 2 * sizeof(float))
@@ -2785,6 +2796,19 @@ int kv_attend_prefill_batch(const kvx_storage *s, uint32_t layer, uint32_t query
   auto st = static_cast<hipStream_t>(stream);
   // Equal chunks (what a scheduler that cuts chunks of its token budget produces) share
   // their launches, 32 sequences at a time; anything else runs sequence by sequence.
+  if (same && by_chunk == n_sequences && n_sequences > 1) {
+    for (uint32_t first = 0; first < n_sequences; first += KVX_LANES_PER_LAUNCH) {
+      const uint32_t count = std::min<uint32_t>(KVX_LANES_PER_LAUNCH, n_sequences - first);
+      const int fast = kvx_prefill_chunk_launch(s, kv, query_heads,
+                                                static_cast<const uint16_t *>(queries) + first * sequence_stride,
+                                                static_cast<uint16_t *>(output) + first * sequence_stride,
+                                                page_tables + first, params + first, count, sequence_stride,
+                                                workspace, st);
+      if (l.head_dim == 256) took(fast);
+      if (fast) return fast;
+    }
+    return KVX_OK;
+  }
   if (alike && n_sequences > 1) {
     int fast = 0;
     for (uint32_t first = 0; first < n_sequences && fast == 0; first += KVX_LANES_PER_LAUNCH) {
