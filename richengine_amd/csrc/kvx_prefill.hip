@@ -48,9 +48,11 @@ struct ChunkArgs {
   kvx_kv_layer kv;
 };
 
-// int4 and bf16 operands are bf16, int8 and e4m3 operands fp16 (each holds the codes exactly).
+// Operands are bf16, on e4m3 pages fp16 (each holds the codes exactly).  int8 codes as fp16 would
+// need the weights as fp16 too, whose places run out below 2^-14: a weight carries its token's value
+// scale, so values of standard deviation 1e-3 would move a row by 1.4e-2.
 template <uint32_t FMT>
-constexpr bool kHalfOperands = FMT == KVX_FMT_INT8 || FMT == KVX_FMT_FP8E4M3;
+constexpr bool kHalfOperands = FMT == KVX_FMT_FP8E4M3;
 
 template <uint32_t FMT>
 __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
@@ -83,11 +85,11 @@ template <bool HIGH>
 __device__ __forceinline__ uint32_t fp8_pair(uint32_t x) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HIGH));
 }
-// 0x64 over the byte c + 128 is the fp16 number 1024 + 128 + c.
-__device__ __forceinline__ uint32_t int8_pair(uint32_t flipped, uint32_t select) {
-  const uint32_t biased = __builtin_amdgcn_perm(0x64646464u, flipped, select);
-  const f16x2 codes = __builtin_bit_cast(f16x2, biased) - f16x2{_Float16(1152.0f), _Float16(1152.0f)};
-  return __builtin_bit_cast(uint32_t, codes);
+// Two int8 codes: a small integer's float, cut to its upper half, is exact.
+template <bool HIGH>
+__device__ __forceinline__ uint32_t int8_pair(uint32_t x) {
+  const int lo = __builtin_amdgcn_sbfe(int(x), HIGH ? 16 : 0, 8), hi = __builtin_amdgcn_sbfe(int(x), HIGH ? 24 : 8, 8);
+  return __builtin_amdgcn_perm(__float_as_uint(float(hi)), __float_as_uint(float(lo)), 0x07060302u);
 }
 // Eight one-byte elements in order.
 template <uint32_t FMT>
@@ -95,9 +97,7 @@ __device__ __forceinline__ u32x4 byte_operand(uint32_t first, uint32_t second) {
   if constexpr (FMT == KVX_FMT_FP8E4M3) {
     return u32x4{fp8_pair<false>(first), fp8_pair<true>(first), fp8_pair<false>(second), fp8_pair<true>(second)};
   } else {
-    const uint32_t a = first ^ 0x80808080u, b = second ^ 0x80808080u;
-    return u32x4{int8_pair(a, 0x04010400u), int8_pair(a, 0x04030402u), int8_pair(b, 0x04010400u),
-                 int8_pair(b, 0x04030402u)};
+    return u32x4{int8_pair<false>(first), int8_pair<true>(first), int8_pair<false>(second), int8_pair<true>(second)};
   }
 }
 
@@ -489,10 +489,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
         } else {
           const f32x2 wide = {p[j], p[j + 1]};
           bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(wide, bf16x2));
-          if constexpr (FMT == KVX_FMT_INT8) {  // rounded to bf16, carried as fp16
-            const f16x2 pair = {_Float16(__uint_as_float(bits << 16)), _Float16(__uint_as_float(bits & 0xffff0000u))};
-            bits = __builtin_bit_cast(uint32_t, pair);
-          }
         }
         weights[i >> 3][(i & 7) / 2 + j / 2] = bits;
       }

@@ -3,8 +3,14 @@ where a workgroup, a wave or a tile is partly filled, every format and head dime
 (rows written directly) and several (merged), histories on and off a page boundary, held to the
 oracle at the bar of every other prefill test (2e-3 a row, bf16 rounding of the row alone being
 1.6e-3 to 2e-3)."""
+import numpy as np
 import pytest
+import torch
 
+from oracle import kvoracle as ko
+from richengine_amd import kvx
+import gpulib as Gp
+import kvtestlib as T
 import test_gpu_attention as A
 from test_gpu_prefill_small_groups import layout  # noqa: F401
 
@@ -29,3 +35,95 @@ def test_shared_pages_match_the_oracle(layout, fmt):  # noqa: F811
     for committed, rows, splits in CASES[layout]:
         print(f"chunk layout={layout} fmt={fmt} committed={committed} rows={rows} splits={splits}", flush=True)
         A.prefill_case(fmt, committed, rows, forced_splits=splits)
+
+
+class Chunk:
+    """A sequence of `committed` tokens and a chunk of `rows` behind them, drawn unit normal;
+    `change(keys, values, queries)` ([H, tokens, D] twice and [H, rows, G, D], floats) may rewrite them
+    before they are stored.  `stale` more tokens lie in the last page behind the chunk."""
+
+    def __init__(self, layout, fmt, committed, rows, splits, change=None, stale=0, score_scale=0.0):
+        self.layout, self.fmt, self.committed, self.rows, self.splits = layout, fmt, committed, rows, splits
+        H, G, D = layout
+        tokens = committed + rows
+        assert stale <= -tokens % 32
+        rng = np.random.default_rng(tokens)
+        k, v = (rng.standard_normal((H, tokens + stale, D)).astype(np.float32) for _ in range(2))
+        q = rng.standard_normal((H, rows, G, D)).astype(np.float32)
+        if change:
+            change(k, v, q)
+        self.tw = Gp.Twin(fmt, H, D, 2, (tokens + 31) // 32)
+        self.pages = self.tw.pages((tokens + 31) // 32, seed=tokens)
+        self.th, self.td = self.tw.tables(self.pages)
+        stride = (tokens + stale + 31) // 32 * 32
+        ck, cv = T.chunk_buffers(k, v, stride)
+        kvx.append(self.tw.dev, 1, Gp.dev(ck), Gp.dev(cv), [self.td],
+                   [kvx.ChunkParams(0, tokens + stale, stride, len(self.pages))], H * stride * D)
+        torch.cuda.synchronize()
+        self.tw.download()
+        self.stride = (rows + 31) // 32 * 32
+        self.q = np.zeros((H, self.stride, G, D), dtype=np.uint16)
+        self.q[:, :rows] = ko.f32_to_bf16(q).reshape(q.shape)
+        self.score_scale = score_scale
+
+    def output(self):
+        H, G, D = self.layout
+        out = torch.full((H, self.stride, G, D), 0x5A5A, dtype=torch.int16, device="cuda")
+        ws = torch.empty(kvx.prefill_workspace_bytes(self.tw.dev, self.rows, H * G, self.splits), dtype=torch.uint8,
+                         device="cuda")
+        kvx.attend_prefill(self.tw.dev, 1, H * G, Gp.dev(self.q), out, self.td,
+                           kvx.PrefillParams(self.committed, self.rows, self.stride, len(self.pages), kvx.KvLayer(),
+                                             self.splits, self.score_scale), ws)
+        torch.cuda.synchronize()
+        return Gp.host_u16(out)[:, :self.rows]
+
+    def check(self, label):
+        """The rows against the oracle's, at the bar of every other prefill test."""
+        H, G, D = self.layout
+        params = ko.PrefillParams(self.committed, self.rows, self.stride, len(self.pages), self.tw.host.layer(1),
+                                  self.splits, self.score_scale)
+        ok, want, want32 = ko.attend_prefill(self.fmt, H, G, D, self.q, self.th, params)
+        assert ok == 1
+        explain = Gp.prefill_explainer(self.fmt, H, G, D, self.q, self.th, self.tw.host.layer(1), self.committed,
+                                       self.rows, self.splits)
+        if self.score_scale:
+            described = explain
+            explain = lambda index: dict(described(index), score_scale=self.score_scale)  # noqa: E731
+        Gp.check_attention(self.output(), want[:, :self.rows], want32[:, :self.rows],
+                           np.ones((H, self.rows), dtype=bool), A.tol(self.fmt), label, explain=explain)
+
+    def close(self):
+        self.tw.close()
+
+
+# a chunk of each head dimension that shares its pages, in one split and in several
+SHARED = [((4, 6, 256), 70, 43, 1), ((4, 6, 256), 500, 301, 7), ((2, 8, 128), 1003, 320, 8),
+          ((8, 4, 64), 777, 131, 9), ((8, 4, 64), 40, 1027, 1), ((4, 5, 128), 0, 2011, 1)]
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED[1:4])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_small_values_keep_their_bits(layout, committed, rows, splits, fmt):
+    """A weight carries its token's value scale: with values of 1e-3 the products lie below 2^-14,
+    where fp16 runs out of places."""
+    def change(k, v, q):
+        v *= 1e-3
+
+    print(f"small values layout={layout} fmt={fmt}", flush=True)
+    case = Chunk(layout, fmt, committed, rows, splits, change)
+    case.check(f"small values layout={layout} fmt={fmt}")
+    case.close()
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED[1:4])
+@pytest.mark.parametrize("fmt", [ko.INT4, ko.INT8, ko.BF16])   # (the fp8 tile's queries are fp16)
+def test_large_queries_stay_finite(layout, committed, rows, splits, fmt):
+    """Queries beyond fp16's 65504, on keys as much smaller."""
+    def change(k, v, q):
+        q *= 1e5
+        k *= 1e-5
+
+    print(f"large queries layout={layout} fmt={fmt}", flush=True)
+    case = Chunk(layout, fmt, committed, rows, splits, change)
+    case.check(f"large queries layout={layout} fmt={fmt}")
+    case.close()
