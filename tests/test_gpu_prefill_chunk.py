@@ -127,3 +127,36 @@ def test_large_queries_stay_finite(layout, committed, rows, splits, fmt):
     case = Chunk(layout, fmt, committed, rows, splits, change)
     case.check(f"large queries layout={layout} fmt={fmt}")
     case.close()
+
+
+def spoiled_and_clean(layout, fmt, committed, rows, splits, row):
+    """The rows of a chunk whose row `row` (rows: the first token behind the chunk, in the same page) has an
+    infinite element 5 in its key and its value, and the rows of the same chunk without it."""
+    stale = min(1, -(committed + rows) % 32)
+
+    def spoil(k, v, q):
+        k[:, committed + row, 5] = v[:, committed + row, 5] = np.inf
+
+    outputs = []
+    for change in (spoil, None):
+        case = Chunk(layout, fmt, committed, rows, splits, change, stale=stale)
+        outputs.append(case.output())
+        case.close()
+    return outputs
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED)
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_a_token_that_a_row_does_not_see_does_not_reach_it(layout, committed, rows, splits, fmt):
+    """A token with an infinite element is stored with an infinite scale; neither a row before it in the chunk
+    nor, once its page is another sequence's, a row that ends before it may change by it.  (An element that
+    is itself no number, on bf16 and e4m3 pages, does reach its own dimension of the rows of its page.)"""
+    others = np.arange(layout[2]) != 5
+    if fmt in (ko.INT4, ko.INT8):
+        others[:] = True
+    for row in (2 * rows // 3, rows):
+        if row == rows and (committed + rows) % 32 == 0:
+            continue
+        print(f"unseen token layout={layout} fmt={fmt} row={row} of {rows}", flush=True)
+        spoiled, clean = spoiled_and_clean(layout, fmt, committed, rows, splits, row)
+        assert np.array_equal(spoiled[:, :row][..., others], clean[:, :row][..., others])
