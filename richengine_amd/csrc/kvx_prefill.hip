@@ -8,11 +8,15 @@
 // 32x32x16 MFMAs: keys x queries gives a lane 16 of its column's 32 scores (a column is a fused
 // row), whose weights are then the other operand of values x weights as they lie in registers.
 //
-// Nothing but the fused row number ties a row to its workgroup: the tile of 8 chunk rows it
-// belongs to gives every column its own pages [begin, end) of the split and its own workspace
-// row, so a workgroup's rows need not end with a tile, and the result of a row is a function of
-// the row's own tile, split count and pages (reference: prefill/paged_attention.metal:7-206,
-// common/paged_attention_tile.h:85-349, common/paged_attention_fp8_tile.h:34-265).
+// Nothing but the fused row number ties a row to its workgroup, whose rows need not end with a tile.
+// The tiles of 8 chunk rows that end in the same page have the same pages [begin, end) of every
+// split, and a wave's rows are all of such tiles: four tiles are whole waves whatever the group, and
+// where the first page's tiles are fewer than four, the rows start up to 24 columns into the first
+// wave.  So a wave takes the pages of its rows' own tiles and no others, and the result of a row is a
+// function of the row's own tile, split count and pages (reference:
+// prefill/paged_attention.metal:7-206, common/paged_attention_tile.h:85-349,
+// common/paged_attention_fp8_tile.h:34-265).  (With waves across such tiles an element that is no
+// number, on bf16 or e4m3 pages, reached rows whose tiles end a page before it: weight 0 times NaN.)
 //
 // Why this shape: every LDS read feeds one 32x32x16 MFMA, so eight waves of 32 rows ask the LDS
 // for a page's 64 KiB at the rate the matrix cores take it, and 32 rows are what leaves room for
@@ -301,11 +305,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   __shared__ __align__(16) u32x4 query_lds[kQueryLds ? kQueryLds : 1][W][64];
 
   // x: (sequence, split, KV head), so that the workgroups that walk the same pages follow one
-  // another at a distance and tend to meet on the same XCD; y: 256 fused rows, the last first
-  // (they see the most pages).
+  // another at a distance and tend to meet on the same XCD; y: 256 columns (fused rows), the last
+  // first (they see the most pages).
   const uint32_t H = a.kv_heads, G = a.group;
   const uint32_t head = blockIdx.x % H, split = blockIdx.x / H % a.splits, sequence = blockIdx.x / (H * a.splits);
-  const uint32_t first_fused = (gridDim.y - 1 - blockIdx.y) * kRows;
   const uint64_t *const table = a.lane[sequence].table;
   const uint32_t committed = a.lane[sequence].committed;
   const float score_scale = default_score_scale(D, a.lane[sequence].score_scale);
@@ -317,62 +320,61 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   };
 
   const uint32_t tiles = (a.rows + T - 1) / T, fused_rows = tiles * T * G;
+  // Column 0 of the launch is fused row -lead.  The chunk's first page has (committed % 32 + 7) / 8
+  // tiles fewer than four; of their columns, whole waves are left out.
+  const uint32_t lead = (committed % kPage + T - 1) / T * T * G % kWaveRows;
 
   // The pages of a tile under this split.
   struct Cut {
-    uint32_t begin, end, written, visible;
+    uint32_t begin, end, written;
   };
   const auto cut_of = [&](uint32_t tile) {
     Cut c;
-    c.visible = committed + min(a.rows, (tile + 1) * T);
-    const uint32_t pages = (c.visible + kPage - 1) / kPage, per = (pages + a.splits - 1) / a.splits;
+    const uint32_t visible = committed + min(a.rows, (tile + 1) * T);
+    const uint32_t pages = (visible + kPage - 1) / kPage, per = (pages + a.splits - 1) / a.splits;
     c.begin = min(pages, split * per);
     c.end = min(pages, c.begin + per);
     c.written = (pages + per - 1) / per;
     return c;
   };
+  // The fused rows of columns first_column .. first_column + columns - 1: [first, last], empty when
+  // first > last.
+  const uint32_t first_column = (gridDim.y - 1 - blockIdx.y) * kRows;
+  const auto first_row_of = [&](uint32_t column) { return max(column, lead) - lead; };
+  const auto last_row_of = [&](uint32_t column) { return int32_t(min(column, lead + fused_rows - 1)) - int32_t(lead); };
   // The workgroup's pages: from the first tile's first to the last tile's last.  Every thread
   // takes the same way out.
-  const uint32_t last_fused = min(fused_rows, first_fused + kRows) - 1;
-  const uint32_t begin = cut_of(first_fused / (T * G)).begin, end = cut_of(last_fused / (T * G)).end;
+  if (first_column >= lead + fused_rows) return;
+  const uint32_t begin = cut_of(first_row_of(first_column) / (T * G)).begin;
+  const uint32_t end = cut_of(last_row_of(first_column + kRows - 1) / (T * G)).end;
   if (begin >= end) return;
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 31u, h = lane >> 5;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Where column n of the wave lies.
+  const uint32_t wave_column = first_column + wave * kWaveRows;
   struct Column {
-    uint32_t fused, row, tile;
+    uint32_t fused, row;
     bool in_tile, live;
   };
   const auto column_of = [&](uint32_t n) {
     Column c;
-    c.fused = first_fused + wave * kWaveRows + n;
+    c.fused = wave_column + n - lead;  // (wraps below row 0)
     c.row = c.fused / G;
-    c.tile = min(c.row / T, tiles - 1);
     c.in_tile = c.fused < fused_rows;
     c.live = c.in_tile && c.row < a.rows;
     return c;
   };
   const Column column = column_of(n);
-  const Cut cut = cut_of(column.tile);
   const bool live = column.live;
-  // A column's tokens of this split; columns without a row see everything (and count for nothing).
-  const auto token_begin = [&](const Column &c, const Cut &cut) { return c.live ? cut.begin * kPage : 0u; };
-  const auto token_end = [&](const Column &c, const Cut &cut) {
-    return c.live ? min(cut.end * kPage, committed + c.row + 1) : UINT32_MAX;
-  };
-  // Pages that every column sees whole need no test.
-  uint32_t whole_from = token_begin(column, cut), whole_to = token_end(column, cut);
-  uint32_t wave_end = live ? cut.end : 0u;
-#pragma unroll
-  for (uint32_t offset = 32; offset; offset >>= 1) {
-    whole_from = max(whole_from, uint32_t(__shfl_xor(int(whole_from), offset)));
-    whole_to = min(whole_to, uint32_t(__shfl_xor(int(whole_to), offset)));
-    wave_end = max(wave_end, uint32_t(__shfl_xor(int(wave_end), offset)));
-  }
-  whole_from = __builtin_amdgcn_readfirstlane(whole_from);
-  whole_to = __builtin_amdgcn_readfirstlane(whole_to);
-  wave_end = __builtin_amdgcn_readfirstlane(wave_end);  // 0: none of the wave's rows is live
+  // The wave's pages: none when none of its rows is live.  All of its rows see the tokens before
+  // whole_to.
+  const uint32_t wave_row = first_row_of(wave_column) / G;
+  const int32_t wave_last = last_row_of(wave_column + kWaveRows - 1);
+  const bool wave_live = wave_column < lead + fused_rows && wave_last >= 0 && wave_row < a.rows;
+  const Cut cut = cut_of(wave_live ? uint32_t(wave_last) / (T * G) : 0);
+  const uint32_t wave_first = cut.begin - begin, wave_pages = wave_live ? cut.end - cut.begin : 0u;  // slots
+  const uint32_t whole_to = committed + wave_row + 1;
 
   // Queries: a lane holds 8 dims of every 16 of its column.
   const uint64_t head_row = (uint64_t(head) * a.stride) * G;
@@ -446,18 +448,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
       for (uint32_t i = 0; i < 16; ++i) s[i] *= score_scale;
     }
     const uint32_t first_token = page * kPage;
-    const bool masked = first_token < whole_from || first_token + kPage > whole_to;
+    const bool masked = first_token + kPage > whole_to;
     uint32_t unseen = 0;  // (of a masked page) bit i: score i
     if (masked) {
       const Column own = column_of(n);  // found again on the few such pages rather than kept
-      const Cut own_cut = cut_of(own.tile);
-      const uint32_t from = token_begin(own, own_cut), to = token_end(own, own_cut);
+      // (columns without a row see everything, and count for nothing)
+      const uint32_t to = own.live ? committed + own.row + 1 : UINT32_MAX;
 #pragma unroll
       for (uint32_t i = 0; i < 16; ++i) {
         const uint32_t token = first_token + 16 * (i >> 3) + 8 * h + (i & 7);
-        const bool outside = token < from || token >= to;
-        if (outside) s[i] = -INFINITY;
-        if constexpr (kQuant) unseen |= outside ? 1u << i : 0u;
+        if (token >= to) s[i] = -INFINITY;
+        if constexpr (kQuant) unseen |= token >= to ? 1u << i : 0u;
       }
     }
     float local_max = fmaxf(s[0], s[1]);
@@ -567,7 +568,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
       stage_share<FMT, D>(staged[next], scale_lds[next], raw, opaque(tid), key_unit);
       fetch_share<FMT, D>(raw, slab_at(slot + (kInt4 ? 4 : 3)), opaque(tid));
     }
-    if (begin + slot < wave_end) attend_page(staged[now], scale_lds[now], begin + slot);
+    if (slot - wave_first < wave_pages) attend_page(staged[now], scale_lds[now], begin + slot);
     if (slot & 1) barrier();
   }
   if constexpr (!kQuant) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the wave
@@ -596,7 +597,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     return v;
   };
   const Column place = column_of(at & 31u);  // found again rather than kept through the loop
-  const Cut cut_again = cut_of(place.tile);
   if (!place.in_tile) return;
   uint16_t *out_row = output + sequence * a.sequence_stride + (head_row + place.fused) * D;
   if (!place.live) {  // rows of the last tile past the live ones read as zeros
@@ -605,8 +605,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
       for (uint32_t k = 0; k < kQuads; ++k) *reinterpret_cast<u32x2 *>(out_row + 8 * k + 4 * half) = u32x2{0u, 0u};
     return;
   }
-  if (cut_again.begin >= cut_again.end) return;
-  if (cut_again.written == 1) {  // one split: the merge's weight is exp(0) = 1
+  if (cut.begin >= cut.end) return;
+  if (cut.written == 1) {  // one split: the merge's weight is exp(0) = 1
     // x / sum by the reciprocal, with the quotient's error put back: the divider's own result
     // but for its last bit, in a third of its instructions.
     const float reciprocal = sum > 0.0f ? __fdiv_rn(1.0f, sum) : 0.0f;
@@ -629,8 +629,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     }
     return;
   }
-  const uint64_t slot_row = sequence * a.sequence_rows + ((uint64_t(place.tile) * H + head) * a.splits + split) * (T * G) +
-                            (place.fused - place.tile * T * G);
+  const uint32_t tile = place.row / T;
+  const uint64_t slot_row = sequence * a.sequence_rows + ((uint64_t(tile) * H + head) * a.splits + split) * (T * G) +
+                            (place.fused - tile * T * G);
   float *part = partials + slot_row * D;
 #pragma unroll
   for (uint32_t k = 0; k < kQuads; ++k) {
@@ -740,9 +741,13 @@ int kvx_prefill_chunk_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t que
   a.kv = kv;
   float *partials = static_cast<float *>(workspace);
   float *statistics = partials + sequences * a.sequence_rows * D;
-  const uint32_t fused = tiles * T * G;
+  // columns: the fused rows behind the kernel's `lead`
+  uint32_t lead = 0;
+  for (uint32_t i = 0; i < sequences; ++i)
+    lead = std::max(lead, (params[i].committed_tokens % KVX_PAGE_TOKENS + T - 1) / T * T * G % kWaveRows);
+  const uint32_t columns = lead + tiles * T * G;
   const auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(H * splits * sequences, (fused + kRows - 1) / kRows),
+    hipLaunchKernelGGL(kernel, dim3(H * splits * sequences, (columns + kRows - 1) / kRows),
                        dim3(kThreads), 0, stream, static_cast<const uint16_t *>(queries),
                        static_cast<uint16_t *>(output), partials, statistics, a);
   };

@@ -160,3 +160,17 @@ def test_a_token_that_a_row_does_not_see_does_not_reach_it(layout, committed, ro
         print(f"unseen token layout={layout} fmt={fmt} row={row} of {rows}", flush=True)
         spoiled, clean = spoiled_and_clean(layout, fmt, committed, rows, splits, row)
         assert np.array_equal(spoiled[:, :row][..., others], clean[:, :row][..., others])
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED + [((3, 5, 128), 1100, 90, 32), ((2, 13, 64), 1090, 61, 32)])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_an_element_that_is_no_number_stays_in_its_pages(layout, committed, rows, splits, fmt):
+    """The first token of a page that begins in the chunk has an infinite element: rows whose tiles end before
+    that page have the bits that they have without it."""
+    first = -committed % 32
+    for row in {first, first + 32 * ((rows - 1 - first) // 32)}:
+        print(f"no number layout={layout} fmt={fmt} row={row} of {rows}", flush=True)
+        spoiled, clean = spoiled_and_clean(layout, fmt, committed, rows, splits, row)
+        before = row // 8 * 8
+        assert before == 0 or np.isfinite(ko.bf16_to_f32(clean[:, :before].copy())).all()
+        assert np.array_equal(spoiled[:, :before], clean[:, :before])
