@@ -278,8 +278,10 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
 }
 // exp(x), x <= 0, to about an ulp: 2^(x log2 e) with the product's rounding error put back.
 __device__ __forceinline__ float exact_exp(float x) {
-  x = fmaxf(x, -1000.0f);  // (of -inf the rounding error would be no number)
-  const float y = x * kLog2e, rest = fmaf(x, kLog2e, -y), e = __builtin_amdgcn_exp2f(y);
+  const float y = x * kLog2e, e = __builtin_amdgcn_exp2f(y);
+  // Of -inf the rounding error is no number, which the median takes for its lower bound: what is 0
+  // stays 0, and of an x that is no number e is none either.
+  const float rest = __builtin_amdgcn_fmed3f(fmaf(x, kLog2e, -y), -1.0f, 1.0f);
   return fmaf(e, rest * 0.693147180559945309f, e);
 }
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32); }
@@ -609,8 +611,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   if (cut.written == 1) {  // one split: the merge's weight is exp(0) = 1
     // x / sum by the reciprocal, with the quotient's error put back: the divider's own result
     // but for its last bit, in a third of its instructions.
-    const float reciprocal = sum > 0.0f ? __fdiv_rn(1.0f, sum) : 0.0f;
+    const bool some = sum > 0.0f;  // a sum that is no number leaves no row, as in the merge
+    const float reciprocal = some ? __fdiv_rn(1.0f, sum) : 0.0f;
     const auto divided = [&](float x) {
+      if (!some) return 0.0f;
       const float quotient = x * reciprocal;
       const float better = fmaf(fmaf(-quotient, sum, x), reciprocal, quotient);
       return fabsf(quotient) < INFINITY ? better : quotient;  // (an infinite quotient has no error)

@@ -174,3 +174,23 @@ def test_an_element_that_is_no_number_stays_in_its_pages(layout, committed, rows
         before = row // 8 * 8
         assert before == 0 or np.isfinite(ko.bf16_to_f32(clean[:, :before].copy())).all()
         assert np.array_equal(spoiled[:, :before], clean[:, :before])
+
+
+# (int4 chunks in one split at head dimension 256 run tile by tile)
+@pytest.mark.parametrize("fmt,layout,committed,rows,splits",
+                         [(f, *c) for f in A.FORMATS for c in SHARED if f != ko.INT4 or c[0][2] != 256 or c[3] > 1])
+def test_a_score_that_is_no_number_leaves_no_row(layout, committed, rows, splits, fmt):
+    """A key with an infinite element against queries that are 0 there: the score is no number, nor is the sum of
+    the weights, and such a row is written as zeros, in one split and in several, at every head dimension."""
+    row = 2 * rows // 3
+
+    def change(k, v, q):
+        k[:, committed + row, 5] = np.inf
+        q[..., 5] = 0.0
+
+    print(f"no score layout={layout} fmt={fmt} row={row} of {rows}", flush=True)
+    case = Chunk(layout, fmt, committed, rows, splits, change)
+    got = case.output()
+    assert not got[:, row:].any()
+    assert got[:, :row].any(axis=-1).all() and np.isfinite(ko.bf16_to_f32(got[:, :row].copy())).all()
+    case.close()
