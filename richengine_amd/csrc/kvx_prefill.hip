@@ -69,12 +69,13 @@ __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
 }
 
 // ---- bytes of a page to operand elements -----------------------------------------------
-// int4 codes become bf16 numbers of code / 512 through e4m3, whose bytes 0 .. 8 are 0 .. 8 / 512 (the
-// subnormals and the first normal) and so on up to 15: one conversion takes two of them.  Keys
-// take the codes themselves, sign and magnitude.  Values take u = code + 8, which is one
-// instruction for eight codes; the 8 / 512 an element they carry too much are taken off the
-// finished row as 8 times the sum of its rounded weights.  (Keys' scores would lose their
-// last bits to such a bias where keys have outlier channels.)
+// int4 codes become bf16 numbers through e4m3, whose bytes 0 .. 8 are 0 .. 8 / 512 (the subnormals
+// and the first normal) and so on up to 15: one conversion takes two of them, and its scale the
+// 512.  (As code / 512 the rest went into the key scales, which overflow at keys of 2e37 and more.)
+// Keys take the codes themselves, sign and magnitude.  Values take u = code + 8, which is one
+// instruction for eight codes; the 8 an element they carry too much are taken off the finished
+// row as 8 times the sum of its rounded weights.  (Keys' scores would lose their last bits to
+// such a bias where keys have outlier channels.)
 constexpr float kNibbleUnit = 512.0f, kNibbleBias = 8.0f;
 // Four codes, a byte each (two's complement nibbles), to e4m3 bytes of sign and magnitude.
 __device__ __forceinline__ uint32_t signed_nibbles(uint32_t x) {
@@ -83,7 +84,7 @@ __device__ __forceinline__ uint32_t signed_nibbles(uint32_t x) {
 }
 template <bool HIGH>
 __device__ __forceinline__ uint32_t nibble_pair(uint32_t bytes) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(bytes, 1.0f, HIGH));
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(bytes, kNibbleUnit, HIGH));
 }
 template <bool HIGH>
 __device__ __forceinline__ uint32_t fp8_pair(uint32_t x) {
@@ -413,9 +414,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     return slab_of(FMT, H, D, a.kv, head, scalar_entry(entries, min(slot, last_slot)));
   };
   PageShare<FMT, D> raw;
-  // What goes into the key scales: powers of two and, but for head dimension 128, whose default is
-  // none, the score scale.
-  const float key_unit = (kInt4 ? kNibbleUnit : 1.0f) * (D == 128 ? 1.0f : score_scale);
+  // What goes into the key scales: the score scale, but for head dimension 128, whose default is no
+  // power of two.
+  const float key_unit = D == 128 ? 1.0f : score_scale;
 
   // A staged page against the wave's rows.
   const auto attend_page = [&](const uint8_t *copy, const float *scales, uint32_t page) __attribute__((always_inline)) {
@@ -589,7 +590,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
 #pragma unroll
       for (uint32_t i = 0; i < 4; ++i) {
         const uint32_t place = r + (first + i) * (D / 8), in_block = place % 32;
-        v[i] = acc[place / 32][(in_block & 3) + 4 * (in_block >> 3)] * kNibbleUnit - bias;
+        v[i] = acc[place / 32][(in_block & 3) + 4 * (in_block >> 3)] - bias;
       }
       dim = 8 * (r + 4 * half) + first;
     } else {

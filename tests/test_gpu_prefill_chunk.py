@@ -194,3 +194,17 @@ def test_a_score_that_is_no_number_leaves_no_row(layout, committed, rows, splits
     assert not got[:, row:].any()
     assert got[:, :row].any(axis=-1).all() and np.isfinite(ko.bf16_to_f32(got[:, :row].copy())).all()
     case.close()
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED[1:])
+def test_int4_keys_near_the_largest_number(layout, committed, rows, splits):
+    """A key element of 2e38 against queries that are 0 there: every other code of the key is 0, and so is its score,
+    whatever the code unit and the score scale are multiplied into."""
+    def change(k, v, q):
+        k[:, committed // 2, 5] = 2e38
+        q[..., 5] = 0.0
+
+    print(f"large key layout={layout} splits={splits}", flush=True)
+    case = Chunk(layout, ko.INT4, committed, rows, splits, change)
+    case.check(f"large key layout={layout}")
+    case.close()
