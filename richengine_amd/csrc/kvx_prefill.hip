@@ -277,14 +277,13 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   asm volatile("" : "+v"(x));
   return x;
 }
-// exp(x), x <= 0: 2^y with y = x log2 e rounded, times 1 + (x - y ln 2), ln 2 in two parts.
+// exp(x), x <= 0, to about an ulp: 2^(x log2 e) with the product's rounding error put back.
 __device__ __forceinline__ float exact_exp(float x) {
-  constexpr float kLn2 = 0.693147180559945309f, kLn2Low = float(0.693147180559945309 - double(kLn2));
   const float y = x * kLog2e, e = __builtin_amdgcn_exp2f(y);
-  // Of -inf the rest is no number, which the median takes for its lower bound: what is 0 stays 0,
-  // and of an x that is no number e is none either.
-  const float rest = __builtin_amdgcn_fmed3f(fmaf(-y, kLn2Low, fmaf(-y, kLn2, x)), -1.0f, 1.0f);
-  return fmaf(e, rest, e);
+  // Of -inf the rounding error is no number, which the median takes for its lower bound: what is 0
+  // stays 0, and of an x that is no number e is none either.
+  const float rest = __builtin_amdgcn_fmed3f(fmaf(x, kLog2e, -y), -1.0f, 1.0f);
+  return fmaf(e, rest * 0.693147180559945309f, e);
 }
 __device__ __forceinline__ float other_half(float x) { return __shfl_xor(x, 32); }
 __device__ __forceinline__ float halves_max(float x) {
