@@ -16,9 +16,15 @@ extern "C" {
    matrix-core (MFMA) kernels, so tests can tell which path they measured. */
 void kvx_debug_attend_paths(uint64_t *generic_calls, uint64_t *matrix_core_calls);
 
-/* How many consecutive 8-row tiles of a kv_attend_prefill call at head dimension 64 or 128 share
-   a workgroup and a staged page (1 = every tile on its own; 0 = invalid arguments), so tests can
-   tell which kernel a chunk ran on. */
+/* Whether a kv_attend_prefill call of these parameters runs as workgroups of 256 fused rows that share
+   their pages (1) or tile by tile (0; also for invalid arguments), so tests can tell which kernel
+   a chunk ran on. */
+uint32_t kvx_debug_prefill_by_chunk(const kvx_layout *layout, uint32_t query_heads,
+                                    uint32_t committed_tokens, uint32_t rows, uint32_t splits);
+
+/* How many consecutive 8-row tiles of a kv_attend_prefill call at head dimension 64 or 128 that runs
+   tile by tile share a workgroup and a staged page (1 = every tile on its own; 0 = invalid
+   arguments), so tests can tell which kernel a chunk ran on. */
 uint32_t kvx_debug_prefill_tiles_together(const kvx_layout *layout, uint32_t query_heads,
                                           uint32_t committed_tokens, uint32_t rows, uint32_t splits);
 

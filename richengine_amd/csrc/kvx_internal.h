@@ -140,26 +140,15 @@ inline uint32_t verify_block_rows(uint32_t format, uint32_t fused_rows) {
   if (format == KVX_FMT_INT4 && 26 * by48 < 15 * by32) return 48;
   return 32;
 }
-// Whether a chunk runs as workgroups of 256 fused rows that share their pages (kvx_prefill.hip)
-// rather than as waves and workgroups of single tiles, which spread a small call over more
-// CUs.  A function of the sequence alone: a batch gives a sequence the bits of its own call.
-// Times are one layer's call, tiles / workgroups of 256:
-//  head dimension 256: bf16, int8 and e4m3 pages in one split always (64 rows after 32 tokens, bf16
-//    32.3 / 17.7 us; 8 rows even or better), under several from 64 rows (64 rows after 512 tokens, fp8
-//    40.1 / 35.2) or 20 000 fused rows of work items on (33 rows over 8192 tokens in 28 splits, bf16
-//    61 / 38; in 2 splits 20.6 / 29.1).  int4 pages under several splits from 40 000 on (over 8192
-//    tokens in 5 splits: 256 rows, 30 720, 117 / 127 us; 512 rows 162 / 140).
-//  64 and 128: from 32 768 and 40 000 on (64 rows over 8192 tokens in 32 splits: 64-wide bf16, 65 536,
-//    33 / 28 us, 128-wide 32 768, 29 / 34; 128 rows 40.4 / 37.8), where the splits hold more than a
-//    page: below, sharing has nothing to share.
-inline bool prefill_by_chunk(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
-  const uint32_t D = l.head_dim, H = l.kv_heads, G = query_heads / H;
-  const uint64_t work = uint64_t(p.rows) * G * H * p.split_count;
-  if (D == 256 && l.format == KVX_FMT_INT4) return p.split_count > 1 && work >= 40000;
-  if (D == 256) return p.split_count == 1 || p.rows >= 64 || work >= 20000;
-  if (D != 64 && D != 128) return false;
-  const uint64_t pages = (uint64_t(p.committed_tokens) + p.rows + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS;
-  return pages > p.split_count && work >= (D == 64 ? 32768u : 40000u);
+// Workgroups of 256 fused rows that share their pages (kvx_prefill.hip): the columns of a chunk's launch
+// before its first fused row.  The first page of the chunk has (committed % 32 + 7) / 8 tiles fewer than
+// four, and a wave of 32 columns is to hold tiles of one page alone; whole waves are left out.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline uint32_t prefill_chunk_lead(uint32_t committed, uint32_t group) {
+  constexpr uint32_t T = KVX_PREFILL_TILE_ROWS;
+  return (committed % KVX_PAGE_TOKENS + T - 1) / T * T * group % 32;
 }
 // Whether tiles 2i and 2i + 1 of a chunked prefill that starts after `committed`
 // tokens see the same number of pages, for every i: tile 2i sees committed + 16 i

@@ -6,6 +6,8 @@
 // left unfused so the fp32 results do not depend on contraction.
 #include <atomic>
 #include <algorithm>
+#include <cmath>
+#include <numeric>
 #include <vector>
 
 #include "kvx_device.h"
@@ -1806,7 +1808,7 @@ int kvx_attend_wide_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t
 
 int kvx_prefill_chunk_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t query_heads,
                              const void *queries, void *output, const uint64_t *const *page_tables,
-                             const kvx_prefill_params *params, uint32_t sequences,
+                             const kvx_prefill_params *params, const uint32_t *at, uint32_t sequences,
                              uint64_t sequence_stride, void *workspace, hipStream_t stream);
 
 // int4 pages go to their own kernels, bf16, fp8 and int8 pages to the wide-element
@@ -2597,6 +2599,87 @@ TileShape tile_shape(const kvx_layout &l, uint32_t query_heads, const kvx_prefil
   return shape;
 }
 
+// ---- tiles, or workgroups of 256 fused rows that share their pages (kvx_prefill.hip)? ----
+// A function of the sequence alone: a batch gives a sequence the bits of its own call.  Both kernels
+// timed on 38 518 calls of one sequence (21 head layouts, all formats, 8 to 2048 rows after 0 to
+// 16 384 tokens, 1 to 32 splits and the plans').
+//
+// bf16, int8 and e4m3 pages of head dimension 256.  In one split a row has the same bits whatever the
+// length of its chunk, so the choice is the layout's: the workgroups, at 0.5 to 0.95 of the tiles' time
+// by format and group over the plans' calls (4 x 6: 33 bf16 rows after 8192 tokens, whose odd tile is a
+// second walk, 607 / 400 us; the worst are even tiles of 2, 8 or 16 heads on e4m3 pages, 256 rows
+// after 8192 tokens at 4 x 2 375 / 503), but for e4m3 pages under groups of one head (1.12, and up to
+// 1.75: 256 rows after 512 tokens at 8 x 1 37 / 65).
+// In several splits what decides is how serial either is (128 rows of e4m3 after 40 tokens in two, which
+// tiles spread over 384 waves: 15.6 / 27.8), so the time of a page of every split is compared: `alone`
+// while the kernel's workgroups (of four waves; single waves count as a quarter) find a CU each, with
+// more of them `full` for each to a CU.  Microseconds, fitted to 10 297 calls: together they take 2 %
+// longer than with the better kernel each time, and 2 % are more than 5 % slower than as tiles (with the
+// workgroups from 64 rows on, whatever the group, it was 19 %).  The history's length does not enter:
+// sequences of a batch that are of two minds do not share their launches.
+struct PageTime {
+  double alone, full;
+  double operator()(double workgroups_per_cu) const { return std::max(alone, full * workgroups_per_cu); }
+};
+double prefill_tiles_page(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
+  constexpr double kCus = 256, kCuWaves = 4 * kCus;
+  const uint32_t H = l.kv_heads, M = KVX_PREFILL_TILE_ROWS * (query_heads / H), splits = p.split_count;
+  const uint32_t tiles = (p.rows + KVX_PREFILL_TILE_ROWS - 1) / KVX_PREFILL_TILE_ROWS;
+  const TileShape shape = tile_shape(l, query_heads, p);
+  const uint32_t lanes = tiles / shape.width, rest = tiles % shape.width, fused = M * shape.width;
+  const bool bf16 = l.format == KVX_FMT_BF16, int8 = l.format == KVX_FMT_INT8;
+  const auto single = [&](uint32_t n) {  // tiles on waves of their own
+    const uint32_t rows = bf16 && M > 16 ? 32 : 16;
+    const double per_cu = double(n) * H * splits * ((M + rows - 1) / rows) / kCuWaves;
+    return (bf16 ? PageTime{1.15, 2.4} : int8 ? PageTime{1.5, 1.45} : PageTime{1.12, 1.4})(per_cu);
+  };
+  if (!lanes) return single(rest);
+  // An odd last tile is a launch of its own, which walks the pages once more.
+  const double after = rest ? (bf16 ? 1.12 : int8 ? 1.5 : 1.13) : 0;
+  if (shape.width == 1) return after + single(lanes);
+  if (shape.lane_kind == 2) {  // a workgroup to a CU
+    const double per_cu = std::ceil(double(lanes) * H * splits / kCus);
+    const bool three = fused > 128;  // blocks of 16 rows to a wave
+    const PageTime page = bf16   ? (three ? PageTime{2.1, 2.35} : PageTime{1.5, 1.65})
+                          : int8 ? (three ? PageTime{2.3, 2.6} : PageTime{1.68, 1.85})
+                                 : (three ? PageTime{2.15, 2.45} : PageTime{1.53, 1.72});
+    return after + (per_cu > 1 ? page.full * per_cu : page.alone);
+  }
+  const bool one_block = fused <= 16;
+  const uint32_t rows = one_block ? 16 : 32;
+  const double per_cu = double(lanes) * H * splits * ((fused + rows - 1) / rows) / kCuWaves, share = one_block ? 0.93 : 1;
+  return after + (bf16 ? PageTime{1.15 * share, 2.5} : int8 ? PageTime{1.65 * share, 1.8} : PageTime{1.3 * share, 1.6})(per_cu);
+}
+double prefill_chunk_page(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
+  const uint32_t H = l.kv_heads, G = query_heads / H;
+  const uint32_t tiles = (p.rows + KVX_PREFILL_TILE_ROWS - 1) / KVX_PREFILL_TILE_ROWS;
+  const uint32_t columns = tiles * KVX_PREFILL_TILE_ROWS * G + kvx::prefill_chunk_lead(p.committed_tokens, G);
+  const double rounds = std::ceil(double((columns + 255) / 256) * H * p.split_count / 256);  // a workgroup to a CU
+  const bool few = columns <= 128;                                                           // a wave to a SIMD
+  return rounds * (l.format == KVX_FMT_BF16   ? (few ? 1.18 : 1.6)
+                   : l.format == KVX_FMT_INT8 ? (few ? 1.52 : 2.0)
+                                              : (few ? 1.46 : 1.95));
+}
+bool prefill_by_chunk(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
+  const uint32_t D = l.head_dim;
+  const uint64_t work = uint64_t(p.rows) * query_heads * p.split_count;
+  const uint64_t pages = (uint64_t(p.committed_tokens) + p.rows + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS;
+  const uint64_t per = (pages + p.split_count - 1) / p.split_count;
+  // int4 pages of head dimension 256 in several splits, and head dimensions 64 and 128: from a launch's
+  // work on, where the tiles fill the GPU.  A sequence alone takes 0.92 of the tiles' time from there on
+  // at 256, 0.80 at 128 and 0.72 at 64 (162 of 1113, 310 of 2180 and 289 of 3884 calls are more than 5 %
+  // slower, of those in the plans' splits one in thirteen or fewer); half of the line at 256 a call takes
+  // 1.24 of it, at 128 1.05, at 64 1.0.  Batches share the workgroups' launches, which the tiles at 64
+  // and 128 do not (four chunks of 290 rows after 1696 tokens in 14 splits at 2 x 8 x 128, int4: 155 /
+  // 108 us).  In splits of a single page a sixth of the calls is slower, by up to 1.6 times: tiles.
+  if (D == 64 || D == 128) return per > 1 && work >= (D == 64 ? 32768u : 40000u);
+  if (D != 256) return false;
+  if (l.format == KVX_FMT_INT4) return p.split_count > 1 && work >= 40000;
+  if (p.split_count == 1) return l.format != KVX_FMT_FP8E4M3 || query_heads > l.kv_heads;
+  if (p.rows < 64 && work < 20000) return false;
+  return prefill_chunk_page(l, query_heads, p) < prefill_tiles_page(l, query_heads, p);
+}
+
 int validate_prefill(const kvx_layout &l, uint32_t query_heads, const kvx_prefill_params &p) {
   const kvx_chunk_params chunk{p.committed_tokens, p.rows, p.chunk_stride, p.page_table_entries, {}};
   static const char *const names[] = {"", "chunk_tokens_out_of_range", "context_out_of_range",
@@ -2674,6 +2757,16 @@ int prefill_matrix(const kvx_storage *s, kvx_kv_layer kv, uint32_t query_heads, 
 }
 }  // namespace
 
+uint32_t kvx_debug_prefill_by_chunk(const kvx_layout *layout, uint32_t query_heads, uint32_t committed_tokens,
+                                    uint32_t rows, uint32_t splits) {
+  if (!kvx_layout_valid(layout) || !query_heads || query_heads % layout->kv_heads) return 0;
+  const kvx_prefill_params p{committed_tokens, rows, (rows + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS * KVX_PAGE_TOKENS,
+                             uint32_t((uint64_t(committed_tokens) + rows + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS),
+                             {}, splits, 0.0f};
+  if (validate_prefill(*layout, query_heads, p)) return 0;
+  return prefill_by_chunk(*layout, query_heads, p) ? 1 : 0;
+}
+
 int kv_attend_prefill(const kvx_storage *s, uint32_t layer, uint32_t query_heads,
                       const void *queries, void *output, const uint64_t *page_table,
                       const kvx_prefill_params *params, void *workspace, uint64_t workspace_bytes,
@@ -2696,11 +2789,11 @@ int kv_attend_prefill(const kvx_storage *s, uint32_t layer, uint32_t query_heads
   if (workspace_bytes < partial_bytes + rows * 2 * sizeof(float))
     return fail(KVX_EINVAL, "prefill attention scratch is smaller than its bound");
   auto st = static_cast<hipStream_t>(stream);
-  if (kvx::prefill_by_chunk(l, query_heads, *params)) {
-    const int fast = kvx_prefill_chunk_launch(s, kv, query_heads, queries, output, &page_table, params, 1, 0,
+  if (prefill_by_chunk(l, query_heads, *params)) {
+    const uint32_t at = 0;
+    const int fast = kvx_prefill_chunk_launch(s, kv, query_heads, queries, output, &page_table, params, &at, 1, 0,
                                               workspace, st);
-    if (D == 256) took(fast);
-    if (fast <= 0) return fast;
+    return D == 256 ? took(fast) : fast;
   }
   {
     const int fast = prefill_matrix(s, kv, query_heads, queries, output, &page_table, params, 1, 0,
@@ -2775,8 +2868,8 @@ int kv_attend_prefill_batch(const kvx_storage *s, uint32_t layer, uint32_t query
   // Nothing is enqueued unless every sequence is valid.
   const uint32_t G = query_heads / l.kv_heads;
   uint64_t rows = 0;
-  bool alike = true, same = true;
-  uint32_t by_chunk = 0;
+  bool same = true;
+  std::vector<uint32_t> by_chunk, by_tile;  // sequences
   for (uint32_t q = 0; q < n_sequences; ++q) {
     if (!page_tables[q]) return fail(KVX_EINVAL, "null page table");
     if (int rc = validate_prefill(l, query_heads, params[q])) return rc;
@@ -2787,47 +2880,50 @@ int kv_attend_prefill_batch(const kvx_storage *s, uint32_t layer, uint32_t query
     same = same && params[q].rows == params[0].rows &&
            params[q].chunk_stride == params[0].chunk_stride &&
            params[q].split_count == params[0].split_count;
-    by_chunk += kvx::prefill_by_chunk(l, query_heads, params[q]) ? 1u : 0u;
-    alike = alike && same && !by_chunk &&
-            tile_shape(l, query_heads, params[q]) == tile_shape(l, query_heads, params[0]);
+    (prefill_by_chunk(l, query_heads, params[q]) ? by_chunk : by_tile).push_back(q);
   }
   if (workspace_bytes < rows * l.head_dim * sizeof(float) + 256 + rows * 2 * sizeof(float))
     return fail(KVX_EINVAL, "prefill attention scratch is smaller than its bound");
   auto st = static_cast<hipStream_t>(stream);
   // Equal chunks (what a scheduler that cuts chunks of its token budget produces) share
   // their launches, 32 sequences at a time; anything else runs sequence by sequence.
-  if (same && by_chunk == n_sequences && n_sequences > 1) {
-    for (uint32_t first = 0; first < n_sequences; first += KVX_LANES_PER_LAUNCH) {
-      const uint32_t count = std::min<uint32_t>(KVX_LANES_PER_LAUNCH, n_sequences - first);
-      const int fast = kvx_prefill_chunk_launch(s, kv, query_heads,
-                                                static_cast<const uint16_t *>(queries) + first * sequence_stride,
-                                                static_cast<uint16_t *>(output) + first * sequence_stride,
-                                                page_tables + first, params + first, count, sequence_stride,
-                                                workspace, st);
+  const auto chunks = [&](const std::vector<uint32_t> &at) {
+    for (size_t first = 0; first < at.size(); first += KVX_LANES_PER_LAUNCH) {
+      const uint32_t count = uint32_t(std::min<size_t>(KVX_LANES_PER_LAUNCH, at.size() - first));
+      const int fast = kvx_prefill_chunk_launch(s, kv, query_heads, queries, output, page_tables, params,
+                                                at.data() + first, count, sequence_stride, workspace, st);
       if (l.head_dim == 256) took(fast);
       if (fast) return fast;
     }
-    return KVX_OK;
+    return 0;
+  };
+  if (same) {
+    if (const int rc = chunks(by_chunk)) return rc;
+    if (by_tile.empty()) return KVX_OK;
   }
-  if (alike && n_sequences > 1) {
-    int fast = 0;
-    for (uint32_t first = 0; first < n_sequences && fast == 0; first += KVX_LANES_PER_LAUNCH) {
-      const uint32_t count = std::min<uint32_t>(KVX_LANES_PER_LAUNCH, n_sequences - first);
-      fast = prefill_matrix(s, kv, query_heads,
-                            static_cast<const uint16_t *>(queries) + first * sequence_stride,
-                            static_cast<uint16_t *>(output) + first * sequence_stride,
-                            page_tables + first, params + first, count, sequence_stride, workspace,
-                            workspace_bytes, st);
-      if (fast > 0 && first) return fail(KVX_ESTATE, "a later part of the batch was declined");
+  // Tile by tile: neighbouring sequences whose tiles go to the kernels alike share their launches.
+  if (!same) by_tile.resize(n_sequences), std::iota(by_tile.begin(), by_tile.end(), 0u);  // every sequence
+  for (size_t i = 0, run; i < by_tile.size(); i += run) {
+    const uint32_t q = by_tile[i];
+    for (run = 1; same && i + run < by_tile.size() && run < KVX_LANES_PER_LAUNCH; ++run)
+      if (by_tile[i + run] != q + run ||
+          !(tile_shape(l, query_heads, params[q + run]) == tile_shape(l, query_heads, params[q])))
+        break;
+    if (run > 1) {
+      const int fast = prefill_matrix(s, kv, query_heads,
+                                      static_cast<const uint16_t *>(queries) + q * sequence_stride,
+                                      static_cast<uint16_t *>(output) + q * sequence_stride, page_tables + q,
+                                      params + q, uint32_t(run), sequence_stride, workspace, workspace_bytes, st);
+      if (fast < 0) return fast;
+      if (fast == 0) continue;
     }
-    if (fast <= 0) return fast;
+    for (uint32_t k = q; k < q + run; ++k)
+      if (int rc = kv_attend_prefill(s, layer, query_heads,
+                                     static_cast<const uint16_t *>(queries) + k * sequence_stride,
+                                     static_cast<uint16_t *>(output) + k * sequence_stride,
+                                     page_tables[k], &params[k], workspace, workspace_bytes, stream))
+        return rc;
   }
-  for (uint32_t q = 0; q < n_sequences; ++q)
-    if (int rc = kv_attend_prefill(s, layer, query_heads,
-                                   static_cast<const uint16_t *>(queries) + q * sequence_stride,
-                                   static_cast<uint16_t *>(output) + q * sequence_stride,
-                                   page_tables[q], &params[q], workspace, workspace_bytes, stream))
-      return rc;
   return KVX_OK;
 }
 

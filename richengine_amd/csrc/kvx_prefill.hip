@@ -42,6 +42,7 @@ struct ChunkLane {
   const uint64_t *table;
   uint32_t committed;
   float score_scale;
+  uint32_t at;  // the sequence's place in queries and output, in sequence strides
 };
 struct ChunkArgs {
   ChunkLane lane[kLanes];
@@ -323,9 +324,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   };
 
   const uint32_t tiles = (a.rows + T - 1) / T, fused_rows = tiles * T * G;
-  // Column 0 of the launch is fused row -lead.  The chunk's first page has (committed % 32 + 7) / 8
-  // tiles fewer than four; of their columns, whole waves are left out.
-  const uint32_t lead = (committed % kPage + T - 1) / T * T * G % kWaveRows;
+  const uint32_t lead = prefill_chunk_lead(committed, G);  // column 0 of the launch is fused row -lead
 
   // The pages of a tile under this split.
   struct Cut {
@@ -381,7 +380,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
 
   // Queries: a lane holds 8 dims of every 16 of its column.
   const uint64_t head_row = (uint64_t(head) * a.stride) * G;
-  const uint16_t *q_row = queries + sequence * a.sequence_stride + (head_row + (live ? column.fused : 0u)) * D;
+  const uint16_t *q_row = queries + a.lane[sequence].at * a.sequence_stride + (head_row + (live ? column.fused : 0u)) * D;
   u32x4 q[kQueryRegs];
 #pragma unroll
   for (uint32_t kb = 0; kb < kSteps; ++kb) {
@@ -601,7 +600,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   };
   const Column place = column_of(at & 31u);  // found again rather than kept through the loop
   if (!place.in_tile) return;
-  uint16_t *out_row = output + sequence * a.sequence_stride + (head_row + place.fused) * D;
+  uint16_t *out_row = output + a.lane[sequence].at * a.sequence_stride + (head_row + place.fused) * D;
   if (!place.live) {  // rows of the last tile past the live ones read as zeros
     if (split == 0)
 #pragma unroll
@@ -713,7 +712,7 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(uint16_t *__restrict__
   for (uint32_t i = 0; i < 2; ++i)
     packed[i] = uint32_t(f32_to_bf16(denominator > 0.0f ? __fdiv_rn(numerator[2 * i], denominator) : 0.0f)) |
                 uint32_t(f32_to_bf16(denominator > 0.0f ? __fdiv_rn(numerator[2 * i + 1], denominator) : 0.0f)) << 16;
-  *reinterpret_cast<u32x2 *>(output + sequence * a.sequence_stride + ((uint64_t(head) * a.stride) * G + fused) * D + 4 * lane) = packed;
+  *reinterpret_cast<u32x2 *>(output + a.lane[sequence].at * a.sequence_stride + ((uint64_t(head) * a.stride) * G + fused) * D + 4 * lane) = packed;
 }
 
 }  // namespace
@@ -721,23 +720,26 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(uint16_t *__restrict__
 
 using namespace kvx;
 
-// The chunks of up to 32 sequences (equal rows, stride and split count) in one launch of
-// each kernel; 1 = declined, 0 when enqueued, or a negative status.  The caller has checked
-// the parameters and the workspace's size (rows x D + 2 floats per workspace row).
+// The chunks of up to 32 sequences (equal rows, stride and split count) in one launch of each
+// kernel: sequences at[0], at[1], .. of the caller's arrays.  0 when enqueued, or a negative status.
+// The caller has checked the parameters, that prefill_by_chunk takes them, and the workspace's
+// size (rows x D + 2 floats per workspace row).
 int kvx_prefill_chunk_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query_heads, const void *queries,
                              void *output, const uint64_t *const *page_tables, const kvx_prefill_params *params,
-                             uint32_t sequences, uint64_t sequence_stride, void *workspace, hipStream_t stream) {
+                             const uint32_t *at, uint32_t sequences, uint64_t sequence_stride, void *workspace,
+                             hipStream_t stream) {
   const kvx_layout &l = s->layout;
   const uint32_t H = l.kv_heads, G = query_heads / H, D = l.head_dim, T = KVX_PREFILL_TILE_ROWS;
-  if ((D != 64 && D != 128 && D != 256) || sequences > kLanes) return 1;
-  const uint32_t rows = params[0].rows, splits = params[0].split_count, tiles = (rows + T - 1) / T;
+  const kvx_prefill_params &first = params[at[0]];
+  const uint32_t rows = first.rows, splits = first.split_count, tiles = (rows + T - 1) / T;
   ChunkArgs a{};
-  for (uint32_t i = 0; i < sequences; ++i)
-    a.lane[i] = {page_tables[i], params[i].committed_tokens,
-                 params[i].score_scale != 0.0f ? params[i].score_scale : l.score_scale};
+  for (uint32_t i = 0; i < sequences; ++i) {
+    const kvx_prefill_params &p = params[at[i]];
+    a.lane[i] = {page_tables[at[i]], p.committed_tokens, p.score_scale != 0.0f ? p.score_scale : l.score_scale, at[i]};
+  }
   a.sequences = sequences;
   a.rows = rows;
-  a.stride = params[0].chunk_stride;
+  a.stride = first.chunk_stride;
   a.splits = splits;
   a.kv_heads = H;
   a.group = G;
@@ -749,7 +751,7 @@ int kvx_prefill_chunk_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t que
   // columns: the fused rows behind the kernel's `lead`
   uint32_t lead = 0;
   for (uint32_t i = 0; i < sequences; ++i)
-    lead = std::max(lead, (params[i].committed_tokens % KVX_PAGE_TOKENS + T - 1) / T * T * G % kWaveRows);
+    lead = std::max(lead, prefill_chunk_lead(a.lane[i].committed, G));
   const uint32_t columns = lead + tiles * T * G;
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(H * splits * sequences, (columns + kRows - 1) / kRows),

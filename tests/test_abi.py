@@ -443,3 +443,34 @@ def test_prefill_plan_by_layout():
     # absurd sizes neither hang nor wrap
     for committed, rows in ((0xFFFFFFFF, 0xFFFFFFFF), (0, 0), (0xFFFFFFFF, 1), (5, 0xFFFFFFFF)):
         assert 0 <= plan(8, 4, 64, committed, rows) <= 32
+
+
+def test_prefill_by_chunk_rule():
+    """kvx_debug_prefill_by_chunk: one split at head dimension 256 by layout and format alone (a row's bits do not
+    depend on the length of its chunk), several where the workgroups of 256 fused rows are no more serial than
+    the tiles, int4 pages and head dimensions 64 and 128 from a launch's work on."""
+    import ctypes as C
+
+    def by_chunk(heads, group, dim, fmt, committed, rows, splits):
+        layout = kvx.Layout(1, heads, dim, fmt, 0.0)
+        return kvx.lib().kvx_debug_prefill_by_chunk(C.byref(layout), heads * group, committed, rows, splits)
+
+    wide = (kvx.BF16, kvx.INT8, kvx.FP8)
+    for fmt in wide:
+        for committed, rows in ((0, 8), (31, 33), (8192, 256), (16384, 2048)):
+            assert by_chunk(4, 6, 256, fmt, committed, rows, 1) == 1
+            assert by_chunk(8, 1, 256, fmt, committed, rows, 1) == (fmt != kvx.FP8)
+            assert by_chunk(4, 6, 256, kvx.INT4, committed, rows, 1) == 0
+        # few rows in few splits: tiles spread over more of the GPU
+        assert by_chunk(4, 6, 256, fmt, 40, 128, 2) == 0 and by_chunk(4, 2, 256, fmt, 4096, 128, 2) == 0
+        assert by_chunk(1, 8, 256, fmt, 1000, 64, 4) == 0
+        # 64 rows of a group of one head are two of a workgroup's eight waves
+        assert by_chunk(8, 1, 256, fmt, 8192, 64, 4) == 0
+        # full launches, and odd tiles that would be a second walk
+        assert by_chunk(4, 6, 256, fmt, 8192, 777, 3) == 1 and by_chunk(4, 6, 256, fmt, 8192, 100, 8) == 1
+    assert by_chunk(4, 6, 256, kvx.INT4, 8192, 512, 4) == 1 and by_chunk(4, 6, 256, kvx.INT4, 8192, 416, 4) == 0
+    assert by_chunk(2, 8, 128, kvx.FP8, 8192, 256, 32) == 1 and by_chunk(2, 8, 128, kvx.FP8, 8192, 64, 32) == 0
+    assert by_chunk(8, 4, 64, kvx.INT4, 8192, 32, 32) == 1 and by_chunk(8, 4, 64, kvx.INT4, 8192, 31, 32) == 0
+    assert by_chunk(8, 4, 64, kvx.INT4, 0, 1024, 32) == 0       # splits of a single page
+    assert by_chunk(4, 6, 192, kvx.BF16, 0, 64, 1) == 0 and by_chunk(4, 0, 256, kvx.BF16, 0, 64, 1) == 0
+    assert by_chunk(4, 6, 256, kvx.BF16, 0, 64, 33) == 0 and by_chunk(4, 6, 256, kvx.BF16, 0, 0, 1) == 0
