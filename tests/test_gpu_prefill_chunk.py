@@ -3,6 +3,8 @@ where a workgroup, a wave or a tile is partly filled, every format and head dime
 (rows written directly) and several (merged), histories on and off a page boundary, held to the
 oracle at the bar of every other prefill test (2e-3 a row, bf16 rounding of the row alone being
 1.6e-3 to 2e-3)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -12,6 +14,7 @@ from richengine_amd import kvx
 import gpulib as Gp
 import kvtestlib as T
 import test_gpu_attention as A
+import test_gpu_prefill_batch as B
 from test_gpu_prefill_small_groups import layout  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -35,6 +38,24 @@ def test_shared_pages_match_the_oracle(layout, fmt):  # noqa: F811
     for committed, rows, splits in CASES[layout]:
         print(f"chunk layout={layout} fmt={fmt} committed={committed} rows={rows} splits={splits}", flush=True)
         A.prefill_case(fmt, committed, rows, forced_splits=splits)
+
+
+def by_chunk(layout, fmt, committed, rows, splits):
+    """Whether the call runs as workgroups of 256 fused rows at all."""
+    H, G, D = layout
+    return bool(kvx.lib().kvx_debug_prefill_by_chunk(C.byref(kvx.Layout(1, H, D, fmt, 0.0)), H * G, committed, rows, splits))
+
+
+def tile_by_tile(layout, fmt, splits):
+    """Of the cases of this file: int4 and, under a group of one head, e4m3 pages in one split at 256."""
+    return layout[2] == 256 and splits == 1 and (fmt == ko.INT4 or (fmt == ko.FP8 and layout[1] == 1))
+
+
+def test_the_cases_run_as_workgroups():
+    cases = [(layout, *case) for layout in CASES for case in CASES[layout]] + SHARED
+    for fmt in A.FORMATS:
+        for layout, committed, rows, splits in cases:
+            assert by_chunk(layout, fmt, committed, rows, splits) != tile_by_tile(layout, fmt, splits)
 
 
 class Chunk:
@@ -176,9 +197,8 @@ def test_an_element_that_is_no_number_stays_in_its_pages(layout, committed, rows
         assert np.array_equal(spoiled[:, :before], clean[:, :before])
 
 
-# (int4 chunks in one split at head dimension 256 run tile by tile)
 @pytest.mark.parametrize("fmt,layout,committed,rows,splits",
-                         [(f, *c) for f in A.FORMATS for c in SHARED if f != ko.INT4 or c[0][2] != 256 or c[3] > 1])
+                         [(f, *c) for f in A.FORMATS for c in SHARED if not tile_by_tile(c[0], f, c[3])])
 def test_a_score_that_is_no_number_leaves_no_row(layout, committed, rows, splits, fmt):
     """A key with an infinite element against queries that are 0 there: the score is no number, nor is the sum of
     the weights, and such a row is written as zeros, in one split and in several, at every head dimension."""
@@ -208,3 +228,49 @@ def test_int4_keys_near_the_largest_number(layout, committed, rows, splits):
     case = Chunk(layout, ko.INT4, committed, rows, splits, change)
     case.check(f"large key layout={layout}")
     case.close()
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED[4:])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_one_split_at_64_and_128_is_written_directly(layout, committed, rows, splits, fmt):
+    print(f"one split layout={layout} fmt={fmt}", flush=True)
+    case = Chunk(layout, fmt, committed, rows, splits)
+    case.check(f"one split layout={layout} fmt={fmt}")
+    case.close()
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", SHARED[:4])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_a_score_scale_of_the_callers(layout, committed, rows, splits, fmt):
+    """No power of two and not the default; at 64 and 256 it goes into the staged key scales."""
+    print(f"score scale layout={layout} fmt={fmt}", flush=True)
+    case = Chunk(layout, fmt, committed, rows, splits, score_scale=0.11)
+    case.check(f"score scale layout={layout} fmt={fmt}")
+    case.close()
+
+
+# the sequences' histories, rows and splits; the last two of sequences that go either way
+BATCHES = [((2, 8, 128), (1003, 640, 1024), 320, 8), ((8, 4, 64), (777, 512, 1000), 131, 9),
+           ((3, 5, 128), (1100, 1500, 1088), 90, 32), ((4, 6, 256), (500, 512, 1000), 301, 7),
+           ((8, 4, 64), tuple(512 + 32 * (i % 5) + i for i in range(35)), 66, 16),
+           ((8, 4, 64), (0, 777, 64, 32, 1024, 0), 131, 9), ((4, 6, 256), (512, 500, 1000, 480, 1024, 1030), 64, 3)]
+
+
+@pytest.mark.parametrize("layout,committed,rows,splits", BATCHES)
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_a_batch_has_the_bits_of_its_sequences_alone(monkeypatch, layout, committed, rows, splits, fmt):
+    """Equal chunks share the workgroups' launches, 32 sequences at a time, whatever their histories; those that
+    run tile by tile do not disturb them."""
+    for name, value in zip(("H", "G", "D", "QH"), (*layout, layout[0] * layout[1])):
+        monkeypatch.setattr(B, name, value)
+    ways = {by_chunk(layout, fmt, c, rows, splits) for c in committed}
+    if (layout, committed, rows, splits) not in BATCHES[-2:]:
+        assert ways == {True}
+    else:
+        assert ways == ({False} if layout[2] == 256 and fmt == ko.INT4 else {True, False})
+    print(f"batch layout={layout} fmt={fmt} sequences={len(committed)} rows={rows} splits={splits}", flush=True)
+    n = len(committed)
+    together, alone, tw = B.run_batch(fmt, list(committed), [rows] * n, [splits] * n)
+    assert np.array_equal(together, alone)
+    assert (alone != 0x5A5A).any(axis=1).all()
+    tw.close()
