@@ -15,7 +15,16 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 #define KVX_GLOBAL __attribute__((address_space(1)))
+
+// Two e4m3 bytes (the low or the high half of x) to two fp16 halves holding their
+// values: one v_cvt_scalef32_pk_f16_fp8 with scale 1.
+template <bool HIGH>
+__device__ __forceinline__ uint32_t fp8_pair(uint32_t x) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HIGH));
+}
 
 // Loads through pointers rebuilt from page entries: say they are global memory
 // so the compiler emits global_load rather than flat_load.

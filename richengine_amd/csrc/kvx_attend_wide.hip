@@ -23,14 +23,12 @@
 // packed fp16 subtraction of 1152 leaves the code itself, exactly.  Queries and
 // probabilities meet the codes as fp16: a bf16 query, or a probability already
 // rounded to bf16 as the reference tile rounds it, converts without loss unless
-// its magnitude is below 2^-14, far under the tolerance.
+// its magnitude is below 2^-14 (a probability carries its token's value scale, so
+// values far below 1 lose places) or above 65504.
 #include "kvx_attend_common.h"
 
 namespace kvx {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 template <uint32_t FMT>
 struct Wide {
@@ -52,12 +50,6 @@ __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Two e4m3 bytes (the low or the high half of x) to two fp16 halves holding their
-// values: one v_cvt_scalef32_pk_f16_fp8 with scale 1.
-template <bool HIGH>
-__device__ __forceinline__ uint32_t fp8_pair(uint32_t x) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HIGH));
-}
 // Eight consecutive bytes (two dwords) to eight fp16 in order.
 __device__ __forceinline__ u32x4 fp8_operand(uint32_t first, uint32_t second) {
   return u32x4{fp8_pair<false>(first), fp8_pair<true>(first), fp8_pair<false>(second),

@@ -177,9 +177,11 @@ inline bool prefill_pairs_with_splits(uint32_t format, uint32_t committed, uint3
   if (format == KVX_FMT_INT4 && tiles < 64) return false;
   return 2ull * prefill_paired_waves(tiles, kv_heads, group) * splits >= prefill_paired_slots(format);
 }
-// What kvx_prefill_plan counts on bf16, fp8 and int8 pages of head dimension 256: chunks from
-// kGroupedPrefillRows rows on as groups of four (or two) tiles, up to 192 fused rows, that share
-// a workgroup and its pages.  0 = no such groups for this shape.
+// bf16, fp8 and int8 pages of head dimension 256, chunks from kGroupedPrefillRows rows on that
+// stay tile by tile: in lanes of four (or two) tiles, for a workgroup of four waves that
+// fetches every page once for all of them and shares it through LDS, where the lane's fused
+// rows fit three blocks of 16 per wave (192).  What kvx_prefill_plan counts.
+// 0 = no such lanes for this shape.
 constexpr uint32_t kGroupedPrefillRows = 64;
 inline uint32_t prefill_group_width(uint32_t format, uint32_t head_dim, uint32_t rows, uint32_t group) {
   if (format == KVX_FMT_INT4 || head_dim != 256 || rows < kGroupedPrefillRows) return 0;
@@ -188,8 +190,9 @@ inline uint32_t prefill_group_width(uint32_t format, uint32_t head_dim, uint32_t
   // Groups of one or two query heads would leave three quarters of every wave's rows empty.
   return width * tile_fused >= 96 ? width : 0u;
 }
-// Whether the tiles of every such group see the same number of pages: groups of four tiles
-// (32 rows) when the chunk starts on a page boundary, groups of two as for pairs.
+// Whether the tiles of every such lane see the same number of pages, so that a lane cut into
+// splits is each of its tiles cut into splits: lanes of four tiles (32 rows) when the chunk
+// starts on a page boundary, lanes of two as for pairs.
 inline bool prefill_group_splits_alike(uint32_t width, uint32_t committed) {
   return width == 4 ? committed % KVX_PAGE_TOKENS == 0 : prefill_tiles_pair(committed);
 }

@@ -2575,6 +2575,8 @@ namespace {
 // splits, which they do when they see the same number of pages
 // (prefill_tiles_pair: true for every pair of the chunk, or for none), and pay
 // only where the paired launch fills the GPU (prefill_pairs_with_splits).
+// bf16, fp8 and int8 pages: lanes of four (or two) tiles for a workgroup that shares
+// every page through LDS (prefill_group_width) where a lane's tiles cut their pages alike.
 struct TileShape {
   uint32_t width;  // tiles per lane
   int lane_kind;   // attend_matrix's many_tiles

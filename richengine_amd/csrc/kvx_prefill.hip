@@ -18,8 +18,9 @@
 // common/paged_attention_fp8_tile.h:34-265).  (With waves across such tiles an element that is no
 // number, on bf16 or e4m3 pages, reached rows whose tiles end a page before it: weight 0 times NaN.)
 //
-// Why this shape: every LDS read feeds one 32x32x16 MFMA, so eight waves of 32 rows ask the LDS
-// for a page's 64 KiB at the rate the matrix cores take it, and 32 rows are what leaves room for
+// Why this shape: every LDS read feeds one 32x32x16 MFMA, so eight waves of 32 rows, each of which
+// reads the whole staged page (32 KiB at head dimension 256), ask the LDS for its 128 bytes a
+// cycle at the rate the matrix cores take them, and 32 rows are what leaves room for
 // two waves a SIMD at head dimension 256 (128 accumulators, 64 queries): one wave's softmax runs
 // under the other's MFMAs.  One wave a SIMD of 48 rows (four to a workgroup) had to take them in
 // turn: 777 bf16 rows after 8192 tokens 632 -> 216 us a layer, of which 129 were the rows left
@@ -31,8 +32,6 @@
 namespace kvx {
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t W = 8, kThreads = 64 * W;              // waves and threads of a workgroup
@@ -86,10 +85,6 @@ __device__ __forceinline__ uint32_t signed_nibbles(uint32_t x) {
 template <bool HIGH>
 __device__ __forceinline__ uint32_t nibble_pair(uint32_t bytes) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(bytes, kNibbleUnit, HIGH));
-}
-template <bool HIGH>
-__device__ __forceinline__ uint32_t fp8_pair(uint32_t x) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HIGH));
 }
 // Two int8 codes: a small integer's float, cut to its upper half, is exact.
 template <bool HIGH>
