@@ -1173,9 +1173,9 @@ def chunked_prefill(args):
         "roofline": {"bound": "mfma", "achieved": round(achieved, 1), "peak": peak, "unit": "TFLOP/s",
                      "frac": round(achieved / peak, 4), "traffic": None,
                      "kernel": ("kv_attend_prefill_batch of one layer: every sequence's tiles in one launch of "
-                                "the split kernel (prefill_int4_kernel or group_wide_kernel)" if batched else
+                                "the split kernel (prefill_int4_kernel or chunk_attend_kernel)" if batched else
                                 "kv_attend_prefill of one sequence and layer: the split kernel (prefill_int4_kernel "
-                                "or group_wide_kernel) and, with several splits, the merge behind it"),
+                                "or chunk_attend_kernel) and, with several splits, the merge behind it"),
                      "flops_per_launch": flops, "ms_per_launch": round(kernel_ms, 4),
                      "sequences_per_launch": launch_sequences,
                      "one_sequence_ms_per_launch": round(single_ms, 4)},
@@ -1414,9 +1414,11 @@ def prefill_layout(args):
     """A chunk of chunked prefill over the reference's other shipped layouts (2 KV heads x 8 x 128,
     8 x 4 x 64) and two with smaller groups of query heads (2 x 4 x 128, 4 x 2 x 128): `--prefill-chunk`
     rows (2048 by default) over 16 384 tokens of history, one sequence, one layer per call, splits
-    from kvx_prefill_plan_for.  Timed on a history that ends on a page boundary, where the tiles that
-    begin in the same page share a workgroup and a staged page, and on the same history plus one
-    token, where every tile runs on its own.  `value` is the matrix-core rate of the first."""
+    from kvx_prefill_plan_for.  Timed on a history that ends on a page boundary and on the same history
+    plus one token.  A chunk of that work runs as workgroups of 256 fused rows either way; one that is
+    too small for them runs tile by tile, where the tiles that begin in the same page share a
+    workgroup and a staged page on the first and every tile runs on its own on the second.  `value` is
+    the matrix-core rate of the first."""
     import numpy as np
     import torch
     from richengine_amd import kvx
@@ -1444,7 +1446,10 @@ def prefill_layout(args):
 
     def timed(committed):
         splits = kvx.prefill_plan_for(storage, committed, rows, query_heads)
-        together = kvx.lib().kvx_debug_prefill_tiles_together(C.byref(layout), query_heads, committed, rows, splits)
+        shape = (C.byref(layout), query_heads, committed, rows, splits)
+        together = kvx.lib().kvx_debug_prefill_tiles_together(*shape)
+        if kvx.lib().kvx_debug_prefill_by_chunk(*shape):
+            together = 256 // (8 * group)
         params = kvx.PrefillParams(committed, rows, rows, n_pages, kvx.KvLayer(), splits, 0.0)
         ws = torch.empty(kvx.prefill_workspace_bytes(storage, rows, query_heads, splits), dtype=torch.uint8,
                          device="cuda")
@@ -1479,8 +1484,8 @@ def prefill_layout(args):
                                              "TFLOPs": round(flops / alone_s / 1e12, 1)},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 1), "peak": peak, "unit": "TFLOP/s",
                      "frac": round(achieved / peak, 4), "traffic": None,
-                     "kernel": "prefill_group_small_kernel / prefill_split_small_kernel + prefill_reduce_kernel "
-                               "(the call; the split kernel is all but a few microseconds of it)",
+                     "kernel": "chunk_attend_kernel + chunk_merge_kernel, or for small chunks prefill_group_small_kernel "
+                               "/ prefill_split_small_kernel + prefill_reduce_kernel (the call)",
                      "flops_per_launch": flops, "ms_per_launch": round(aligned_s * 1e3, 4)},
         "cpu_baseline": None,
     }

@@ -181,9 +181,11 @@ uint32_t kvx_decode_splits(uint32_t committed_tokens, uint32_t rows);
 int kvx_decode_plan(const uint32_t *committed_tokens, uint32_t n_lanes, uint32_t kv_heads,
                     uint32_t format, uint32_t *split_counts);
 /* kvx_prefill_plan_batch by layout: head dimension 256 is that plan; at head dimensions 64 and
-   128 (runtime/ops/PagedAttention.cpp:66-115), whose tiles run a workgroup each, or one for the
-   four or two tiles that begin in the same page of a chunk on a page-aligned history, the fewest
-   splits that make 4096 workgroups, none shorter than 4 pages, at most KVX_PREFILL_MAX_SPLITS.
+   128 (runtime/ops/PagedAttention.cpp:66-115) the fewest splits that make 4096 workgroups, none
+   shorter than 4 pages, at most KVX_PREFILL_MAX_SPLITS, counted as the tiles would run: a
+   workgroup each, or one for the four or two tiles that begin in the same page of a chunk on a
+   page-aligned history.  (Most chunks under that plan run as workgroups of 256 fused rows, see
+   kv_attend_prefill; the plan does not count those, nor the sequences of a batch.)
    0 for an invalid layout, bad head counts or no sequences. */
 uint32_t kvx_prefill_plan_for(const kvx_layout *layout, uint32_t committed_tokens, uint32_t rows,
                               uint32_t query_heads, uint32_t n_sequences);
@@ -234,7 +236,9 @@ int kvx_chunk_validation(const kvx_chunk_params *params);
    8 x group <= 48 fused rows, or two of <= 96, one workgroup per lane, split and KV head, one
    workgroup per CU): one split where those workgroups fill three quarters of the 256 CUs, else
    the count (same bounds) that fills them, where the chunk starts on a page boundary (lanes
-   of two tiles: where the tiles pair); other starts fall under the rules above.
+   of two tiles: where the tiles pair); other starts fall under the rules above.  The counts are
+   those of chunks that run tile by tile, also where kv_attend_prefill takes workgroups of 256
+   fused rows.
    Returns 0 for bad head counts.  No counterpart in the reference (its rule is
    kvx_prefill_splits); any count in 1..32 is valid for kv_attend_prefill. */
 uint32_t kvx_prefill_plan(uint32_t committed_tokens, uint32_t rows, uint32_t kv_heads,
@@ -720,7 +724,11 @@ int kv_append_attend_decode_hidden(const kvx_storage *storage, uint32_t layer, c
    causal over committed + its rows.  Replaces ops::PagedAttention::addPrefill
    (PagedAttention.cpp:442-465; kernels prefill/paged_attention.metal:7-206).
    queries / output: bf16 [kv head][chunk_stride][group][D].  workspace: at
-   least kvx_prefill_workspace() partials + statistics. */
+   least kvx_prefill_workspace() partials + statistics.
+   A chunk runs tile by tile, or as workgroups of 256 fused rows (row x query head of the
+   group) that share their pages, whichever suits its layout, rows and splits.  The two sum
+   in different orders, so the bits of a row, which is within the same bounds either way, can
+   depend on the length of its chunk; in one split at head dimension 256 they do not. */
 int kv_attend_prefill(const kvx_storage *storage, uint32_t layer, uint32_t query_heads,
                       const void *queries, void *output, const uint64_t *page_table,
                       const kvx_prefill_params *params, void *workspace,
@@ -729,9 +737,10 @@ int kv_attend_prefill(const kvx_storage *storage, uint32_t layer, uint32_t query
    command (ops::PagedAttention::addVerify's lane array, runtime/ops/PagedAttention.cpp:467-500; its
    addPrefill takes one sequence).  Sequence q has params[q] and page_tables[q]; its queries and
    output rows ([kv head][chunk_stride][group][D] as above) begin q x sequence_stride elements after
-   the first sequence's.  Chunks of the same shape (rows, chunk_stride and split_count equal, and
-   committed_tokens such that their tiles are paired or grouped alike: page-aligned starts always
-   are) share their launches, 32 sequences at a time: every sequence's tiles are lanes of one
+   the first sequence's.  Chunks of the same shape (rows, chunk_stride and split_count equal) share
+   their launches, 32 sequences at a time: those that run as workgroups of 256 fused rows with each
+   other, and at head dimension 256 neighbours that run tile by tile where their tiles are paired or
+   grouped alike (page-aligned starts always are): every sequence's tiles are lanes of one
    launch.  Anything else runs sequence by sequence on `stream`.  Either way every sequence's
    rows are the bits kv_attend_prefill gives for it alone.  workspace: at least the sum of the
    sequences' kvx_prefill_workspace_for() bounds plus 256 bytes.  Nothing is enqueued unless every
