@@ -52,7 +52,7 @@ def run_batch(fmt, committed, rows, splits, poison=0x5A5A):
 
 @pytest.mark.parametrize("fmt", FORMATS)
 @pytest.mark.parametrize("committed,rows,planned", [
-    ((1024, 2048, 512), 264, False),   # one split: paired (int4) or grouped lanes and an odd last tile
+    ((1024, 2048, 512), 264, False),   # one split: paired lanes and an odd last tile (int4), or workgroups of 256 fused rows
     ((1024, 2048, 512), 136, True),    # several splits by kvx_prefill_plan
     ((0, 4096), 2048, False),          # whole chunks, as the bench's prefill step has them
     ((1500, 2524, 476), 130, False),   # starts 4 tokens before a page boundary, rows not a multiple of 8

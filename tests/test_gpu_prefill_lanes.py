@@ -1,11 +1,10 @@
-"""Chunks of 64 rows and more on bf16, fp8 and int8 pages run in lanes of several 8-row tiles
-whose four waves share every page through LDS; shorter chunks run a wave per tile or pair of
-tiles.  Both walk the pages of a row in the same order with the same arithmetic, so a long
-chunk in one call must give, bit for bit, the rows of the same chunk attended in pieces of
-56 rows.  Verify lanes of more than 64 fused rows (bf16 pages: more than 32) run on the same kernels;
+"""In one split chunks on bf16, fp8 and int8 pages run as workgroups of 256 fused rows whatever their
+length, so a long chunk in one call must give, bit for bit, the rows of the same chunk attended in
+pieces of 56 rows, whose rows lie in other waves and workgroups.  Under several splits chunks run so or
+tile by tile, from 64 rows on in lanes of several 8-row tiles whose four waves share every page
+through LDS.  Verify lanes of more than 64 fused rows (bf16 pages: more than 32) run on the same kernels;
 the layouts of tests/test_gpu_attention.py and tests/test_gpu_geometries.py give them 64, 96 and 128
-rows, the most a verify lane may hold.  The pieces are the path that tests/test_gpu_attention.py holds against the
-oracle.  Under several splits every split rounds its weights against its own running maximum,
+rows, the most a verify lane may hold.  Under several splits every split rounds its weights against its own running maximum,
 so those results are held against the oracle with the same splits instead."""
 import numpy as np
 import pytest
@@ -41,7 +40,7 @@ def attend(tw, td, n_pages, heads, group, q, committed, rows, splits):
                          [(fmt, heads, group, 1000, 296)
                           for fmt in (ko.INT8, ko.BF16) for heads, group in [(8, 3), (2, 12), (4, 2)]])
 def test_long_chunk_is_its_short_pieces(fmt, heads, group, committed, rows):
-    # 296 rows: 37 tiles, so lanes of four (or two) tiles and an odd tile on its own;
+    # 296 rows: 37 tiles, the last workgroup and wave partly filled;
     # 1000 tokens before the chunk: its tiles start in the middle of a page
     tw = Gp.Twin(fmt, heads, D, 2, (committed + rows + 31) // 32)
     pages, th, td = A.fill(tw, committed + rows, seed=committed + rows + group)
@@ -69,8 +68,8 @@ def test_long_chunk_is_its_short_pieces(fmt, heads, group, committed, rows):
                                        (4, 6, 0, 256, 8), (4, 6, 1000, 264, 2)]] +
                          [(ko.FP8, 4, 6, 1024, 136, 3)])
 def test_long_chunk_under_several_splits_matches_oracle(fmt, heads, group, committed, rows, splits):
-    # after 1024 and 0 tokens the tiles of a lane cut their pages into the same splits and the
-    # lanes of several tiles run; after 1000 they do not, and the chunk runs tile by tile
+    # after 1024 and 0 tokens the tiles of a lane cut their pages into the same splits, after 1000 they
+    # do not; which of the kernels runs is the rule's (tests/test_abi.py)
     saved = (A.H, A.G, A.QH)
     A.H, A.G, A.QH = heads, group, heads * group
     try:
