@@ -124,6 +124,7 @@ struct DecodeArgs {
   // Work items in the grid's y and KV heads in its x (the heads of an item are dispatched
   // side by side and the items in the order of the lane records) instead of items in x.
   uint32_t item_major;
+  uint32_t items;  // work items of the launch
 };
 
 // The lane with this index of a launch: read from the arguments, or derived
@@ -477,6 +478,7 @@ int launch_matrix_attention(SplitKernel split_kernel, const char *name, uint32_t
       max_splits = std::max(max_splits, p.split_count);
     }
     if (tile_rows) items = n_lanes * lanes[0].split_count;
+    a.items = items;
     if (epilogue && !epilogue->hidden) {
       a.all_partials = 1;
     } else if (epilogue) {
@@ -494,7 +496,9 @@ int launch_matrix_attention(SplitKernel split_kernel, const char *name, uint32_t
                              ? (waves_per_group > 1
                                     ? dim3((H * items + waves_per_group - 1) / waves_per_group, 1, column_blocks)
                                     : dim3(H, items, column_blocks))
-                             : dim3((items + waves_per_group - 1) / waves_per_group, H, column_blocks),
+                             : waves_per_group > 1
+                                   ? dim3((H * items * column_blocks + waves_per_group - 1) / waves_per_group)
+                                   : dim3(items, H, column_blocks),
                          dim3(threads), 0, stream, static_cast<const uint16_t *>(queries),
                          static_cast<uint16_t *>(output), partials, statistics, a);
       const hipError_t e = hipGetLastError();

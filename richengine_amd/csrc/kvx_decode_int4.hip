@@ -416,7 +416,7 @@ __device__ __forceinline__ void append_decode_token(const LaunchArgs &a, const D
 }
 
 // Register sets of pages per wave: two rotate in the one-block decode kernel
-// (two waves per SIMD), one in the three-block verify kernel.
+// (two waves per SIMD), one in the kernels of several row blocks.
 constexpr uint32_t kDecodeDepth = 2;
 constexpr uint32_t kVerify48Depth = 1;
 
@@ -530,29 +530,39 @@ __device__ __forceinline__ void write_blocks(const State *st, const uint32_t *m,
 // kItemMajor: the launch has its work items in the grid's y and the KV heads in x
 // (DecodeArgs::item_major), and its lanes are plain lane records, never the regular tiles of a
 // prefill.
-// kQuad: workgroups of four waves, each wave a work item of its own (items 4 x .. 4 x + 3); the
-// waves share nothing.  A kernel built for two waves per SIMD but launched with at most one
-// wave per SIMD is not always given one SIMD per wave: after another kernel the dispatcher has
-// put two single-wave workgroups on one SIMD of a CU and none on its neighbour (38 of 960
-// SIMDs, the launch 157 instead of 121 us).  The four waves of one workgroup go to the four
-// SIMDs of its CU.
+// kQuad: workgroups of four waves, each with work of its own; the waves share nothing.  Item-major
+// launches deal (item, head) pairs, others (block of rows, item, head), the blocks fastest: the waves
+// that walk the same pages are then on the same CU at about the same time and find them in its
+// caches.  (Dealt by the grid's z they are on different ones: 2048 rows over 4 x 16 384 tokens 34.0 against
+// 32.7 ms in 8 layers; verify steps are within 1 % either way, waves of 16 rows alone lose up to a quarter.)
+// Four waves also go to the four SIMDs of a CU: a kernel built for two waves per SIMD but launched
+// with at most one wave per SIMD is not always given one SIMD per wave: after another kernel the
+// dispatcher has put two single-wave workgroups on one SIMD of a CU and none on its neighbour (38 of 960
+// SIMDs, the launch 157 instead of 121 us).
 template <uint32_t NB, uint32_t kDepth, bool kReused = false, bool kItemMajor = false, bool kQuad = false>
 __device__ __forceinline__ void attend_int4(const uint16_t *__restrict__ queries,
                                             uint16_t *__restrict__ output,
                                             float *__restrict__ partials,
                                             float *__restrict__ statistics, const DecodeArgs &args) {
-  // The forms that have a SIMD to themselves: three blocks, or two with two page sets.
-  constexpr bool kPinned = NB == 3 || (NB == 2 && kDepth >= 2);
-  // Two blocks with one page set run two waves per SIMD with every accumulator in the first
+  // The form that has a SIMD to itself: three blocks.
+  constexpr bool kPinned = NB == 3;
+  // Two blocks run two waves per SIMD with every accumulator in the first
   // register file: they hold their tiles transposed, which needs the rescaling for a quarter
   // of a tile's registers on a fifth of the pages instead of all of them on half.
-  constexpr bool kRowsDown = NB == 2 && kDepth == 1;
+  constexpr bool kRowsDown = NB == 2;
   const uint32_t wave = kQuad ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0u;
-  // item-major workgroups of four waves: (item, head) pairs in dispatch order, heads fastest
-  const uint32_t flat = 4 * blockIdx.x + wave;
-  uint32_t item = kItemMajor ? (kQuad ? 0u : blockIdx.y) : kQuad ? flat : blockIdx.x;
+  const uint32_t flat = 4 * blockIdx.x + wave;  // kQuad: the wave's number in dispatch order
+  uint32_t item = kItemMajor ? (kQuad ? 0u : blockIdx.y) : blockIdx.x;
   uint32_t head = kItemMajor ? (kQuad ? 0u : blockIdx.x) : blockIdx.y;
-  uint32_t li;
+  uint32_t row_block = blockIdx.z, li;
+  if constexpr (kQuad && !kItemMajor) {
+    const uint32_t blocks = (args.fused_rows + 16 * NB - 1) / (16 * NB), pair = flat / blocks;
+    row_block = flat - pair * blocks;
+    // (waves of 16 rows, short splits: the heads of an item side by side, whose slabs of a page are)
+    head = NB == 1 ? pair % args.kv_heads : pair / args.items;
+    item = NB == 1 ? pair / args.kv_heads : pair - head * args.items;
+    if (head >= args.kv_heads || item >= args.items) return;
+  }
   DecodeLane l;
   LaunchArgs a;
   if constexpr (kItemMajor) {
@@ -648,7 +658,7 @@ __device__ __forceinline__ void attend_int4(const uint16_t *__restrict__ queries
   Sight sight[NB];
 #pragma unroll
   for (uint32_t nb = 0; nb < NB; ++nb) {
-    m[nb] = 16 * (NB * blockIdx.z + nb) + t;
+    m[nb] = 16 * (NB * row_block + nb) + t;
     const uint32_t query_row = m[nb] / G;
     in_tile[nb] = m[nb] < M;
     live_row[nb] = in_tile[nb] && query_row < l.active_rows;
@@ -829,51 +839,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   attend_int4<1, kDecodeDepth, false, true, true>(queries, output, partials, statistics, a);
 }
 
-// The same for the 8-row tiles of a chunked prefill with several splits: every
-// tile of the chunk walks the same pages, so the loads may stay in the caches.
+// More than 16 fused rows: a page is walked by several waves, which its loads may stay in the caches
+// for.  A wave of 16 rows expands every page for itself and is three to a SIMD, a wave of 32 shares what
+// it expands between two blocks, and is two to a SIMD with every accumulator in the first
+// register file, where its rescaling costs one instruction a register (235 vector instructions per block
+// and page).  int4_blocks has which one a launch takes.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void verify_int4_kernel(
+    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
+    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
+  attend_int4<1, 1, true, false, true>(queries, output, partials, statistics, a);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void verify32_int4_kernel(
+    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
+    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
+  attend_int4<2, 1, true, false, true>(queries, output, partials, statistics, a);
+}
+// Single tiles of a chunked prefill, and pairs of no more than 16 fused rows: a wave to a workgroup with
+// two register sets of pages (as waves of verify_int4_kernel 256 rows after 8192 tokens in five splits
+// took 168 us instead of 133, one tile after 40 000 in sixteen 143 instead of 99).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_int4_tiles_kernel(
     const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
     float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
   attend_int4<1, kDecodeDepth, true>(queries, output, partials, statistics, a);
 }
-
-// Two blocks per wave share every expanded key and value operand (verify, tree
-// verify, prefill tiles); the accumulators of both take the register file of a
-// whole SIMD lane, so one wave per SIMD.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void verify_int4_kernel(
+// Pairs of tiles in waves of 32 rows: verify32_int4_kernel under a name of its own in a trace.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_int4_kernel(
     const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
     float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
-  attend_int4<2, 2>(queries, output, partials, statistics, a);
+  attend_int4<2, 1, true, false, true>(queries, output, partials, statistics, a);
 }
 
-// The same two blocks with one register set of pages, which fits two waves per
-// SIMD: for the paired tiles of a chunked prefill, whose 1536 waves per 2048-row
-// chunk then all run at once instead of in a full round and a half-empty one
-// (2.0 -> 1.5 ms on 2048 rows over 16K tokens); its page loads may stay in the
-// caches, because every tile of the chunk walks the same pages.  Verify batches, sized to one
-// wave per SIMD by their plan, are faster with two sets and the SIMD to
-// themselves.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_int4_kernel(
-    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
-    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
-  attend_int4<2, 1, true>(queries, output, partials, statistics, a);
-}
-
-// Two blocks with one register set of pages, for lanes of more than 32 fused rows that fill
-// blocks of 32 better than blocks of 48 (a tree of 16 nodes for a group of 6: three waves of
-// 32 rows).  Built for two waves per SIMD, so that every accumulator lives in the first
-// register file, where its rescaling costs one instruction a register instead of three;
-// per block and page it issues 235 vector instructions where the three-block kernel
-// issues 268, and a wave's vector instructions are what these kernels wait for.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void verify32_int4_kernel(
-    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
-    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
-  attend_int4<2, 1, false, false, true>(queries, output, partials, statistics, a);
-}
-
-// Three blocks (48 fused rows: a chain of 8 rows for a group of 6 query heads, half
-// of a 16-node tree) read and expand every page once for all of them; one register set of pages,
-// one wave per SIMD.
+// Three blocks (48 fused rows: a chain of 8 rows for a group of 6 query heads) read and expand every
+// page once for all of them; one register set of pages, one wave per SIMD.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void verify48_int4_kernel(
     const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
     float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
@@ -926,6 +923,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 using namespace kvx;
 
+// Fused rows to a wave, for lanes of more than 16.
+// 16 where the launch's waves then are all on the GPU at once (three to a SIMD) and no split is longer
+// than 48 pages (32 with three to a SIMD: chains of 8 over 32 x 512 .. 16 384 tokens, 37 pages, 133 us, as 48 rows
+// 128): twice the waves of 32 rows, each through its page in half the time, and a GPU that
+// waves of 32 leave half empty is full (chains of 6 rows over 2 x 1000 tokens 20.8 -> 12.4 us, trees of 16
+// nodes over 4 x 8192 47 -> 40, chains of 8 over 32 x 2000 51 -> 42).  Along a longer split the waves
+// of a page drift apart and it comes from memory more than once: 6 waves of 16 rows against 3 of 32 over 4 x
+// 65 536 tokens in 21 splits of 98 pages 204 against 190 us (45 pages: 94 / 94).  There, or with more waves, 32;
+// or 48 where that leaves clearly fewer waves (verify_block_rows) over such long splits (chains of 8 over
+// 16 x 30 000 tokens 173 us, with 32 rows 187; splits of 37 pages and fewer: 125 / 112).
+// The pairs of tiles of a prefill find their pages in the caches whatever their split's length, and are
+// bound by their instructions: 16 rows while that is a wave to a SIMD (512 rows after 512 tokens 74 -> 50 us,
+// two sequences of 300 after 4096 232 -> 171; with 1216 waves of 16 at 2 x 16 x 256 257 us, as 608 of 32 240).
+static uint32_t int4_blocks(uint32_t kv_heads, uint32_t fused_rows, const kvx_verify_params *lanes,
+                            uint32_t n_lanes, bool tiles) {
+  uint64_t waves = 0;
+  uint32_t longest = 0;
+  const uint32_t launched = tiles ? n_lanes : std::min(n_lanes, kLanes);  // of the first launch
+  for (uint32_t i = 0; i < launched; ++i) {
+    const uint64_t pages = (uint64_t(lanes[i].committed_tokens) + lanes[i].active_rows + kPage - 1) / kPage;
+    longest = std::max(longest, uint32_t((pages + lanes[i].split_count - 1) / lanes[i].split_count));
+    waves += uint64_t(lanes[i].split_count) * kv_heads * ((fused_rows + 15) / 16);
+  }
+  if (tiles) return waves <= 1024 ? 16 : 32;
+  if (longest > (waves > 2048 ? 32 : 48)) return verify_block_rows(KVX_FMT_INT4, fused_rows);
+  return waves <= 3072 ? 16 : 32;
+}
+
 // Runs paged attention (split kernel, then the merge of multi-split lanes) for
 // int4 pages of head dimension 256; returns 1 (declined) for shapes it does not
 // cover so the caller runs the format-generic kernels, 0 when enqueued, or a
@@ -950,37 +975,24 @@ int kvx_attend_int4_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
   // The kernel appends the step's token itself only where one wave owns a
   // (sequence, KV head, split): one-row decode.
   if (fused && (fused_rows > 16 || lanes[0].row_capacity != 1)) return 1;
-  // Sharing the expanded operands between two blocks pays where the lanes are few
-  // and long (verify: 13% on 4 x 65536 tokens x 16 tree rows); chunked prefill has
-  // hundreds of tiles of 48 fused rows, where a half-empty second wave and one
-  // wave per SIMD cost more than the sharing saves.
-  if (fused_rows > 16 && !many_tiles && tile_rows)
-    return launch_matrix_attention(prefill_int4_kernel, "prefill_int4_kernel", 32, 64, s, kv,
-                                   query_heads, queries, output, page_tables, lanes, n_lanes,
-                                   row_masks, row_stride, lane_stride, workspace, workspace_bytes,
-                                   stream, nullptr, tile_rows, epilogue);
-  // 48 fused rows per wave where that leaves clearly fewer waves: the pages are
-  // read and expanded once per 48 rows instead of once per 32.
-  if (verify_block_rows(KVX_FMT_INT4, fused_rows) == 48 && !many_tiles)
-    return launch_matrix_attention(verify48_int4_kernel, "verify48_int4_kernel", 48, 64, s, kv,
-                                   query_heads, queries, output, page_tables, lanes, n_lanes,
-                                   row_masks, row_stride, lane_stride, workspace, workspace_bytes,
-                                   stream, nullptr, tile_rows, epilogue);
-  if (fused_rows > 32 && !many_tiles)
-    return launch_matrix_attention(verify32_int4_kernel, "verify32_int4_kernel", 32, 256, s, kv,
-                                   query_heads, queries, output, page_tables, lanes, n_lanes,
-                                   row_masks, row_stride, lane_stride, workspace, workspace_bytes,
-                                   stream, nullptr, tile_rows, epilogue, false, /*waves_per_group=*/4);
-  if (fused_rows > 16 && !many_tiles)
-    return launch_matrix_attention(verify_int4_kernel, "verify_int4_kernel", 32, 64, s, kv,
-                                   query_heads, queries, output, page_tables, lanes, n_lanes,
-                                   row_masks, row_stride, lane_stride, workspace, workspace_bytes,
-                                   stream, nullptr, tile_rows, epilogue);
-  if (tile_rows && !fused)
+  if (tile_rows && !fused && (many_tiles || fused_rows <= 16))
     return launch_matrix_attention(decode_int4_tiles_kernel, "decode_int4_tiles_kernel", 16, 64, s,
                                    kv, query_heads, queries, output, page_tables, lanes, n_lanes,
                                    row_masks, row_stride, lane_stride, workspace, workspace_bytes,
                                    stream, nullptr, tile_rows, epilogue);
+  if (fused_rows > 16) {
+    const uint32_t rows = int4_blocks(s->layout.kv_heads, fused_rows, lanes, n_lanes, tile_rows);
+    if (rows == 48)
+      return launch_matrix_attention(verify48_int4_kernel, "verify48_int4_kernel", 48, 64, s, kv,
+                                     query_heads, queries, output, page_tables, lanes, n_lanes,
+                                     row_masks, row_stride, lane_stride, workspace, workspace_bytes,
+                                     stream, nullptr, tile_rows, epilogue);
+    return launch_matrix_attention(rows == 16 ? verify_int4_kernel : tile_rows ? prefill_int4_kernel : verify32_int4_kernel,
+                                   "int4 kernels of several row blocks", rows, 256, s, kv, query_heads,
+                                   queries, output, page_tables, lanes, n_lanes, row_masks, row_stride,
+                                   lane_stride, workspace, workspace_bytes, stream, nullptr, tile_rows,
+                                   epilogue, false, /*waves_per_group=*/4);
+  }
   // two waves on most SIMDs (of the first launch's lanes): the form whose placement holds
   uint64_t first_waves = 0;
   for (uint32_t i = 0; i < std::min(n_lanes, kLanes); ++i)
