@@ -125,7 +125,15 @@ struct DecodeArgs {
   // side by side and the items in the order of the lane records) instead of items in x.
   uint32_t item_major;
   uint32_t items;  // work items of the launch
+  // The rows are those of several sequences over a common prefix: a row's queries lie row_pitch elements
+  // from the row's before (0: group x head dimension, side by side) and it sees the committed tokens only.
+  uint32_t committed_only;
+  uint64_t row_pitch;
 };
+// Where a fused row's queries lie behind the first row's.
+__device__ __forceinline__ uint64_t query_at(const DecodeArgs &a, uint32_t group, uint32_t row, uint32_t fused) {
+  return a.row_pitch ? row * a.row_pitch + (fused - row * group) * kD : uint64_t(fused) * kD;
+}
 
 // The lane with this index of a launch: read from the arguments, or derived
 // from the first for regular lanes.
@@ -479,6 +487,10 @@ int launch_matrix_attention(SplitKernel split_kernel, const char *name, uint32_t
     }
     if (tile_rows) items = n_lanes * lanes[0].split_count;
     a.items = items;
+    if (epilogue && epilogue->row_pitch) {
+      a.committed_only = 1;
+      a.row_pitch = epilogue->row_pitch;
+    }
     if (epilogue && !epilogue->hidden) {
       a.all_partials = 1;
     } else if (epilogue) {

@@ -511,10 +511,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES
 // pages; each wave keeps its quarter of one page in flight.  An operand read from LDS must
 // feed two row blocks: four waves reading one block's worth each would ask the LDS for
 // twice what it delivers.
-// The same with two waves per workgroup, each fetching half a page, serves verify batches of
-// 33 to 96 fused rows per lane (a chain of 8 rows or a tree of 16 nodes for a group of 6):
-// the one-wave kernels give such a lane two or three waves that each read every page, and
-// on these formats the reading is what they wait for.
+// (Verify lanes of more than 32 fused rows ran on it too, the forms with two waves, two register sets
+// or two copies below; they are verify_lane_kernel's now but for bf16 lanes of more than 96 rows.)
 constexpr uint32_t kGroupWaves = 4;
 
 // The workgroup's barrier between pairs of pages: a wave's LDS writes are done (the LDS
@@ -983,10 +981,30 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
   }
 }
 
+// No launch takes these forms any more; tests/test_abi.py still holds the registers and scratch memory they
+// compile to.
+#define KVX_HELD(...)                                                                                  \
+  template __global__ void group_wide_kernel<__VA_ARGS__>(const uint16_t *__restrict__, uint16_t *__restrict__, \
+                                                          float *__restrict__, float *__restrict__, DecodeArgs);
+KVX_HELD(KVX_FMT_INT8, 2, 4, false, 2)
+KVX_HELD(KVX_FMT_FP8E4M3, 2, 4, false, 2)
+KVX_HELD(KVX_FMT_INT8, 2, 2, false, 1, 2)
+KVX_HELD(KVX_FMT_FP8E4M3, 2, 2, false, 1, 2)
+KVX_HELD(KVX_FMT_BF16, 2, 2, false, 1, 2)
+KVX_HELD(KVX_FMT_BF16, 3, 2, false, 1, 2)
+#undef KVX_HELD
+
 }  // namespace
 }  // namespace kvx
 
 using namespace kvx;
+
+int kvx_verify_lane_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t query_heads,
+                           const void *queries, void *output, const uint64_t *const *page_tables,
+                           const kvx_verify_params *lanes, uint32_t n_lanes,
+                           const uint32_t *row_masks, uint32_t row_stride, uint64_t lane_stride,
+                           void *workspace, uint64_t workspace_bytes, hipStream_t stream,
+                           const kvx::Epilogue *epilogue);
 
 // Runs paged attention for bf16 or fp8 pages of head dimension 256 on the
 // matrix cores; returns 1 (declined) for shapes it does not cover, 0 when
@@ -1032,23 +1050,16 @@ int kvx_attend_wide_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
     if (M > 32u * kGroupWaves) return KVX_GROUP_FORMATS(3, 4, true);
     return KVX_GROUP_FORMATS(2, 4, true);
   }
-  // Verify lanes of more than 32 fused rows: the waves that the lane needs anyway share its
-  // pages.  33 .. 64 rows (a chain of 8 for a group of 6): two waves that fetch half a page
-  // each, with two LDS copies so that two such workgroups fit a CU (batch of 32: bf16 706 ->
-  // 400 us, int8 435 -> 387 us, fp8 405 -> 343 us; with four copies, one workgroup per CU and
-  // half of the SIMDs empty, the byte formats took 550 - 650 us).  65 .. 128 rows (a tree of 16
-  // nodes): four waves over four copies, the byte formats with two sets of page registers
-  // (batch 4 x 65 536 tokens: int8 436 -> 282 us); bf16 up to 96 rows as two waves of 48, which
-  // its direct loads leave the registers for (456 -> 212 us; four waves of 24: 238 us; the
-  // byte formats spill in that form).
-  // A verify lane holds 128 fused rows at most.
-  if (!tile_rows && !many_tiles && M > 32 && M <= 32u * kGroupWaves) {
-    if (format == KVX_FMT_BF16)
-      return M > 96   ? KVX_GROUP(KVX_FMT_BF16, 2, 4, false)
-             : M > 64 ? KVX_GROUP(KVX_FMT_BF16, 3, 2, false, 1, 2)
-                      : KVX_GROUP(KVX_FMT_BF16, 2, 2, false, 1, 2);
-    if (format == KVX_FMT_INT8) return M > 64 ? KVX_GROUP(KVX_FMT_INT8, 2, 4, false, 2) : KVX_GROUP(KVX_FMT_INT8, 2, 2, false, 1, 2);
-    return M > 64 ? KVX_GROUP(KVX_FMT_FP8E4M3, 2, 4, false, 2) : KVX_GROUP(KVX_FMT_FP8E4M3, 2, 2, false, 1, 2);
+  // Verify lanes of more than 32 fused rows, which hold 128 at most, and the rows of sequences over a prefix they
+  // share: waves that multiply beside waves that stage.  (Few workgroups are as fast, 16 lanes of 1200 tokens at
+  // 108 rows 30.1 / 28.8 us, so bf16 lanes of more than 96 rows take four waves of 32 rows here too; over 40 lanes
+  // of 1875 .. 3750 tokens, 112 rows, in the four waves of group_wide_kernel 99 us, in these 102.)
+  const bool shared_prefix = epilogue && epilogue->row_pitch;
+  if (!tile_rows && !many_tiles && (M > 32 || shared_prefix) && M <= 32u * kGroupWaves) {
+    if (format != KVX_FMT_BF16 || M <= 96 || shared_prefix)
+      return kvx_verify_lane_launch(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, row_masks,
+                                    row_stride, lane_stride, workspace, workspace_bytes, stream, epilogue);
+    return KVX_GROUP(KVX_FMT_BF16, 2, 4, false);
   }
 #undef KVX_GROUP_FORMATS
 #undef KVX_GROUP

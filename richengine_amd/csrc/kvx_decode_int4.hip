@@ -668,6 +668,7 @@ __device__ __forceinline__ void attend_int4(const uint16_t *__restrict__ queries
         live_row[nb] ? min(visible, l.committed + min(query_row, l.active_rows - 1) + 1) : visible;
     sight[nb].tree = live_row[nb] && l.masks != nullptr;
     sight[nb].mask = sight[nb].tree ? l.masks[query_row] : 0u;
+    if (!kItemMajor && live_row[nb] && args.committed_only) sight[nb].tree = true;  // (with no bit set)
   }
   const uint32_t db = kPage * H * kRowBytes, sb = kPage * H * 4;
   const RegionOffsets ro = region_offsets(a.kv.extent_pages, db, sb);
@@ -697,6 +698,7 @@ __device__ __forceinline__ void attend_int4(const uint16_t *__restrict__ queries
 #pragma unroll
   for (uint32_t nb = 0; nb < NB; ++nb) {
     const uint16_t *q_row = q_head + uint64_t(live_row[nb] ? m[nb] : 0) * kD;
+    if constexpr (!kItemMajor) q_row = q_head + (live_row[nb] ? query_at(args, G, m[nb] / G, m[nb]) : 0u);
 #pragma unroll
     for (uint32_t kb = 0; kb < 8; ++kb)
       q_raw[nb][kb] = load_global<u32x4>(q_row + 8 * (16 * (kb >> 2) + 4 * g + (kb & 3)));

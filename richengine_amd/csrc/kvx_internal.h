@@ -93,6 +93,9 @@ struct Epilogue {
   uint16_t *hidden;
   bool partials_only = false;
   bool merge_only = false;
+  // Of a lane over a prefix that several sequences share: elements from a row's queries to the next
+  // row's; its rows see the committed tokens only.  0 = ordinary lanes.
+  uint64_t row_pitch = 0;
 };
 
 // Regular lanes of a launch (the tiles of chunked prefill): `rows` > 0 says that the lanes
