@@ -174,13 +174,6 @@ __device__ __forceinline__ DecodeLane lane_of_item(const DecodeArgs &a, uint32_t
   }
   return lane_at(a, index);
 }
-// What a fused append brings to a launch (host side).
-struct FusedAppend {
-  const void *keys, *values;
-  uint64_t lane_stride;
-  uint32_t stride;
-};
-
 // Which tokens one fused query row (an MFMA column) may see
 // (reference: common/paged_attention_tile.h:141-143).
 struct Sight {

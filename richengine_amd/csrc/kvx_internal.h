@@ -98,6 +98,13 @@ struct Epilogue {
   uint64_t row_pitch = 0;
 };
 
+// What a fused append brings to a launch (host side).
+struct FusedAppend {
+  const void *keys, *values;
+  uint64_t lane_stride;
+  uint32_t stride;
+};
+
 // Regular lanes of a launch (the tiles of chunked prefill): `rows` > 0 says that the lanes
 // passed are `sequences` runs of equally many lanes, lane i of a run being its first lane
 // moved on by i x rows query rows and committed tokens over the run's one page table; the

@@ -1805,7 +1805,7 @@ int kvx_attend_wide_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t
                            const uint32_t *row_masks, uint32_t row_stride, uint64_t lane_stride,
                            void *workspace, uint64_t workspace_bytes, int many_tiles,
                            hipStream_t stream, Tiles tile_rows = 0,
-                           const Epilogue *epilogue = nullptr);
+                           const Epilogue *epilogue = nullptr, const FusedAppend *fused = nullptr);
 
 int kvx_prefill_chunk_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t query_heads,
                              const void *queries, void *output, const uint64_t *const *page_tables,
@@ -2528,6 +2528,12 @@ int append_attend_decode(const kvx_storage *s, uint32_t layer, const void *chunk
                                            chunk_keys, chunk_values, chunk_lane_stride, chunk_stride, 0,
                                            epilogue);
   if (fused <= 0) return took(fused);
+  // bf16, e4m3 and int8 pages of head dimension 256 too.
+  const FusedAppend token{chunk_keys, chunk_values, chunk_lane_stride, chunk_stride};
+  const int wide = kvx_attend_wide_launch(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr,
+                                          row_stride, lane_stride, workspace, workspace_bytes, 0,
+                                          static_cast<hipStream_t>(stream), 0, epilogue, &token);
+  if (wide <= 0) return took(wide);
   // Every other shape: the two entries one after the other.
   std::vector<kvx_chunk_params> chunks(n_lanes);
   for (uint32_t i = 0; i < n_lanes; ++i)
