@@ -10,7 +10,7 @@
 #include <numeric>
 #include <vector>
 
-#include "kvx_device.h"
+#include "kvx_small_args.h"
 #include "kvx_debug.h"
 
 namespace kvx {
@@ -593,27 +593,6 @@ __global__ __launch_bounds__(256) void append_page_kernel(const uint16_t *__rest
 }
 
 // ===================================================== generic attention ====
-// One tile = row_capacity query rows x `group` query heads of one KV head
-// (M fused rows) over the pages of one split.
-struct AttendLane {
-  const uint64_t *table;
-  uint32_t committed, entries, split_count, active_rows;
-  uint64_t row_base;   // first fused row of this lane's slots in the workspace
-  uint64_t q_offset;   // element offset of the lane's queries / output
-  uint32_t mask_offset;
-  float score_scale;
-};
-struct AttendArgs {
-  AttendLane lane[kLanes];
-  uint32_t n_lanes;
-  uint32_t kv_heads, group, head_dim;
-  uint32_t row_capacity;
-  uint32_t row_stride;  // rows between KV heads in queries / output
-  kvx_kv_layer kv;
-  // The merge's second output (see Epilogue), from the launch's first lane on.
-  uint16_t *hidden;
-  const uint16_t *packed_qkv;
-};
 struct PrefillArgs {
   const uint64_t *table;
   uint32_t committed, rows, stride, entries, splits;
@@ -622,14 +601,6 @@ struct PrefillArgs {
   kvx_kv_layer kv;
 };
 
-__device__ inline bool attend_contract(const AttendLane &l, const AttendArgs &a) {
-  return l.active_rows > 0 && l.active_rows <= a.row_capacity &&
-         l.entries >= (uint64_t(l.committed) + l.active_rows + kPage - 1) / kPage &&
-         a.kv.extent_pages > 0 &&
-         uint64_t(l.committed) + l.active_rows <= uint64_t(KVX_MAX_PHYSICAL_TOKENS) &&
-         l.split_count > 0 &&
-         l.split_count <= (a.row_capacity == 1 ? KVX_DECODE_MAX_SPLITS : KVX_VERIFY_MAX_SPLITS);
-}
 __device__ inline bool prefill_contract(const PrefillArgs &p) {
   return p.rows > 0 && p.rows <= KVX_PREFILL_TOKEN_BUDGET && p.stride >= p.rows &&
          p.stride <= KVX_PREFILL_TOKEN_BUDGET && p.stride % kPage == 0 &&
@@ -1807,6 +1778,10 @@ int kvx_attend_wide_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t
                            hipStream_t stream, Tiles tile_rows = 0,
                            const Epilogue *epilogue = nullptr, const FusedAppend *fused = nullptr);
 
+bool kvx_decode_small_covers(uint32_t format, uint32_t head_dim, uint32_t group);
+int kvx_decode_small_launch(uint32_t format, const void *queries, float *partials, float *statistics,
+                            const AttendArgs &a, uint32_t max_splits, const FusedAppend *fused, hipStream_t stream);
+
 int kvx_prefill_chunk_launch(const kvx_storage *storage, kvx_kv_layer kv, uint32_t query_heads,
                              const void *queries, void *output, const uint64_t *const *page_tables,
                              const kvx_prefill_params *params, const uint32_t *at, uint32_t sequences,
@@ -2071,7 +2046,8 @@ static int attend_generic(const kvx_storage *s, kvx_kv_layer kv, uint32_t query_
                           const void *queries, void *output, const uint64_t *const *page_tables,
                           const kvx_verify_params *lanes, uint32_t n_lanes,
                           const uint32_t *row_masks, uint32_t row_stride, void *workspace,
-                          hipStream_t stream, const Epilogue *epilogue = nullptr) {
+                          hipStream_t stream, const Epilogue *epilogue = nullptr,
+                          const FusedAppend *fused = nullptr) {
   // The generic split kernel always writes partial rows; the phases are its two launches.
   const uint32_t phases = (epilogue && epilogue->merge_only ? 0u : 1u) |
                           (epilogue && epilogue->partials_only ? 0u : 2u);
@@ -2117,7 +2093,16 @@ static int attend_generic(const kvx_storage *s, kvx_kv_layer kv, uint32_t query_
       max_splits = std::max(max_splits, p.split_count);
     }
     int rc = KVX_OK;
-    if ((phases & 1u) && (D == 64 || D == 128) && M <= 64 * kSmallBlocks)
+    // `fused` comes only with lanes of the first kind.
+    if ((phases & 1u) && capacity == 1 && !row_masks && kvx_decode_small_covers(l.format, D, G)) {
+      FusedAppend token;
+      if (fused)
+        token = {static_cast<const uint16_t *>(fused->keys) + uint64_t(first) * fused->lane_stride,
+                 static_cast<const uint16_t *>(fused->values) + uint64_t(first) * fused->lane_stride, fused->lane_stride,
+                 fused->stride};
+      rc = kvx_decode_small_launch(l.format, queries, partials, statistics, a, max_splits, fused ? &token : nullptr,
+                                   stream);
+    } else if ((phases & 1u) && (D == 64 || D == 128) && M <= 64 * kSmallBlocks)
       rc = dispatch_format(l.format, [&](auto fmt) {
         // head dimensions 64 and 128: the tile on the matrix cores
         const auto launch = [&](auto kernel) {
@@ -2534,6 +2519,12 @@ int append_attend_decode(const kvx_storage *s, uint32_t layer, const void *chunk
                                           row_stride, lane_stride, workspace, workspace_bytes, 0,
                                           static_cast<hipStream_t>(stream), 0, epilogue, &token);
   if (wide <= 0) return took(wide);
+  // The lanes of decode_small_kernel too.
+  if (kvx_decode_small_covers(s->layout.format, s->layout.head_dim, group)) {
+    took(1);
+    return attend_generic(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr, row_stride,
+                          workspace, static_cast<hipStream_t>(stream), epilogue, &token);
+  }
   // Every other shape: the two entries one after the other.
   std::vector<kvx_chunk_params> chunks(n_lanes);
   for (uint32_t i = 0; i < n_lanes; ++i)
