@@ -1229,7 +1229,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(BL
                                row_masks ? row_masks + l.mask_offset : nullptr, l.score_scale);
 }
 
-// Tiles of at most 16 fused rows: a wave per (split, KV head, lane), PRIVATE of them to a
+// Verify tiles of at most 16 fused rows: a wave per (split, KV head, lane), PRIVATE of them to a
 // workgroup (the staged values take 9.3 KiB a wave at head dimension 128).
 template <uint32_t D>
 constexpr uint32_t kSmallPrivateWaves = D == 128 ? 2 : 4;
