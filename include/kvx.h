@@ -180,14 +180,12 @@ uint32_t kvx_decode_splits(uint32_t committed_tokens, uint32_t rows);
 #define KVX_DECODE_MAX_SPLITS 512u
 int kvx_decode_plan(const uint32_t *committed_tokens, uint32_t n_lanes, uint32_t kv_heads,
                     uint32_t format, uint32_t *split_counts);
-/* The split count of a chunk by layout (runtime/ops/PagedAttention.cpp:66-115), for `sequences` chunks
-   of one kv_attend_prefill_batch call after `committed_tokens` each (their mean): where chunks run as
-   workgroups of 256 fused rows (see kv_attend_prefill), the count in which they are fastest by an
-   estimate of their rounds, pages and merge, no split shorter than 4 pages, at most
-   KVX_PREFILL_MAX_SPLITS.  Elsewhere, and for int4 pages of head dimension 256, and of 64 and 128 for
-   one sequence: kvx_prefill_plan_batch at head dimension 256; at 64 and 128 the fewest splits that make
-   4096 workgroups of tiles, a workgroup each, or one for the four or two tiles that begin in the same
-   page of a chunk on a page-aligned history.
+/* kvx_prefill_plan_batch by layout: head dimension 256 is that plan; at head dimensions 64 and
+   128 (runtime/ops/PagedAttention.cpp:66-115) the fewest splits that make 4096 workgroups, none
+   shorter than 4 pages, at most KVX_PREFILL_MAX_SPLITS, counted as the tiles would run: a
+   workgroup each, or one for the four or two tiles that begin in the same page of a chunk on a
+   page-aligned history.  (Most chunks under that plan run as workgroups of 256 fused rows, see
+   kv_attend_prefill; the plan does not count those, nor the sequences of a batch.)
    0 for an invalid layout, bad head counts or no sequences. */
 uint32_t kvx_prefill_plan_for(const kvx_layout *layout, uint32_t committed_tokens, uint32_t rows,
                               uint32_t query_heads, uint32_t n_sequences);

@@ -1,12 +1,10 @@
 // Host side of libkvx: layout geometry, planning rules, extent storage and the
 // page pool.  No kernels here; device memory is reached through the HIP runtime.
 #include "kvx_internal.h"
-#include "kvx_debug.h"
 
 #include <algorithm>
 #include <vector>
 #include <chrono>
-#include <cmath>
 #include <cstring>
 #include <limits>
 #include <numeric>
@@ -338,55 +336,11 @@ int kvx_decode_plan(const uint32_t *committed, uint32_t n_lanes, uint32_t kv_hea
                           format, split_counts + first);
   return KVX_OK;
 }
-// What a chunk's launch takes as workgroups of 256 fused rows (kvx_prefill.hip) in `splits`, in
-// microseconds: a workgroup is its set-up and the pages of its split, one fits a CU (two at head
-// dimension 64), those that see the most are dispatched first and each takes the place that is free
-// next; then the merge, by the partial rows written and read.  Fitted to 12 shapes of each layout and
-// format (one to four sequences, 32 to 2048 rows after 32 to 16 384 tokens) in every split count.
-static double prefill_chunk_time(const kvx_layout &l, uint64_t committed, uint32_t rows, uint32_t group,
-                                 uint32_t sequences, uint32_t splits) {
-  constexpr uint32_t kKinds = 8;  // lengths told apart among the chunk's workgroups
-  const uint32_t D = l.head_dim, T = KVX_PREFILL_TILE_ROWS;
-  const bool bf16 = l.format == KVX_FMT_BF16, int4 = l.format == KVX_FMT_INT4;
-  const double page = D == 256 ? (bf16 ? 1.45 : 1.8) : D == 128 ? (bf16 ? 1.2 : int4 ? 1.6 : 1.45)
-                                                                : (bf16 ? 1.3 : int4 ? 1.9 : 1.5);
-  const double columns = std::ceil(double((uint64_t(rows) + T - 1) / T * T) * group / 256);
-  // (when a place is free, how many of them)
-  const double all_places = D == 64 ? 512.0 : 256.0;
-  std::vector<std::pair<double, double>> places{{0.0, all_places}};
-  const uint32_t kinds = uint32_t(std::min<double>(kKinds, columns));
-  double last = 0;
-  for (uint32_t k = kinds; k--;) {
-    const double here = std::floor(columns * (k + 1) / kinds) - std::floor(columns * k / kinds);
-    const uint64_t tokens = committed + uint64_t(double(rows) * (k + 1) / kinds);
-    const double pages = std::ceil(double((tokens + KVX_PAGE_TOKENS - 1) / KVX_PAGE_TOKENS) / splits);
-    const double length = (D == 256 ? 11.0 : 2.0) + pages * page;
-    double left = here * l.kv_heads * splits * sequences;
-    // (of very many equal ones, whole rounds at once)
-    const double skipped = std::max(0.0, std::floor(left / all_places) - 64);
-    for (auto &p : places) p.first += skipped * length;
-    left -= skipped * all_places;
-    while (left > 0) {
-      const auto first = std::min_element(places.begin(), places.end());
-      const double end = first->first + length, taken = std::min(left, first->second);
-      left -= taken;
-      first->second -= taken;
-      if (first->second <= 0) places.erase(first);
-      const auto same = std::find_if(places.begin(), places.end(), [&](const auto &p) { return p.first == end; });
-      if (same != places.end()) same->second += taken;
-      else places.emplace_back(end, taken);
-      last = std::max(last, end);
-    }
-  }
-  if (splits == 1) return last;
-  const double megabytes = double(splits) * rows * group * l.kv_heads * sequences * D * 8e-6;
-  return last + (D == 256 ? 7.0 + 0.10 * megabytes : 12.0 + 0.165 * megabytes);
-}
-// The split count of a chunk's tiles.
-static uint32_t prefill_tiles_plan(const kvx_layout &l, uint32_t committed, uint32_t rows, uint32_t query_heads,
-                                   uint32_t sequences) {
-  if (l.head_dim != 64 && l.head_dim != 128)
-    return kvx_prefill_plan_batch(committed, rows, l.kv_heads, query_heads, l.format, sequences);
+uint32_t kvx_prefill_plan_for(const kvx_layout *layout, uint32_t committed, uint32_t rows,
+                              uint32_t query_heads, uint32_t sequences) {
+  if (!kvx_layout_valid(layout) || !query_heads || query_heads % layout->kv_heads || !sequences) return 0;
+  if (layout->head_dim != 64 && layout->head_dim != 128)
+    return kvx_prefill_plan_batch(committed, rows, layout->kv_heads, query_heads, layout->format, sequences);
   // Head dimensions 64 and 128: a workgroup of four waves per (tile or group of tiles, KV head,
   // split), four of them to a CU at a time.  The fewest splits that make four rounds of them
   // (4096 workgroups), none shorter than 4 pages (2048 rows over 16 384 tokens, int4, in 1 / 2 /
@@ -397,53 +351,13 @@ static uint32_t prefill_tiles_plan(const kvx_layout &l, uint32_t committed, uint
   if (!tiles) return 1;
   const uint64_t seen = pages_of(uint64_t(committed) + rows / 2);
   const uint32_t most = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(seen / 4, KVX_PREFILL_MAX_SPLITS)));
-  const uint32_t group = query_heads / l.kv_heads;
+  const uint32_t group = query_heads / layout->kv_heads;
   for (uint32_t s = 1; s < most; ++s) {
     const uint32_t together =
-        kvx::small_prefill_tiles_together(l.head_dim, l.kv_heads, group, committed, rows, s);
-    if ((tiles + together - 1) / together * l.kv_heads * s >= 4096) return s;
+        kvx::small_prefill_tiles_together(layout->head_dim, layout->kv_heads, group, committed, rows, s);
+    if ((tiles + together - 1) / together * layout->kv_heads * s >= 4096) return s;
   }
   return most;
-}
-uint32_t kvx_prefill_plan_for(const kvx_layout *layout, uint32_t committed, uint32_t rows,
-                              uint32_t query_heads, uint32_t sequences) {
-  if (!kvx_layout_valid(layout) || !query_heads || query_heads % layout->kv_heads || !sequences) return 0;
-  const kvx_layout &l = *layout;
-  const uint32_t tiles = prefill_tiles_plan(l, committed, rows, query_heads, sequences);
-  const uint32_t group = query_heads / l.kv_heads;
-  if (!tiles || !rows || rows > KVX_PREFILL_TOKEN_BUDGET || KVX_PREFILL_TILE_ROWS * group > 128 ||
-      uint64_t(committed) + rows > KVX_MAX_PHYSICAL_TOKENS)
-    return tiles;
-  const uint64_t seen = pages_of(uint64_t(committed) + rows / 2);
-  const uint32_t most = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(seen / 4, KVX_PREFILL_MAX_SPLITS)));
-  // Fewer than 64 rows at head dimension 256: tiles in a few splits, which run beside one another (37 int8 rows
-  // after 416 tokens 45 us as one workgroup's walk, 18 in three splits; four such e4m3 chunks 51 and 27; two
-  // int4 chunks of 39 rows after 384 tokens 67 in one split, 21 in two).
-  if (l.head_dim == 256 && rows < 64) return std::max(tiles, std::min(3u, most));
-  // Chunks that run as workgroups of 256 fused rows: as many splits as are fastest by their time.
-  // Counted as tiles (a batch's as if one after the other) a bf16 chunk of 2048 rows after 16 384 tokens
-  // at 4 x 6 x 256 had one split, 192 workgroups on 256 CUs (848 us; in four, three full rounds, 680), two
-  // e4m3 chunks of 256 rows after 6144 at 2 x 8 x 128 had 32 (100 us; in 16 73) and three int8 chunks of
-  // 700 rows after 4096 there 24 (325 us; in 5 170).  int4 keeps the tiles' count at head dimension 256,
-  // where a chunk in one split runs tile by tile, and for a sequence alone, whose count the tests of this
-  // function hold: 0.77 to 1 of the time is to be had there (256 rows after 8192 tokens at 2 x 8 x 128
-  // 72 us in 32 splits, 56 in 16).
-  if (l.format == KVX_FMT_INT4 && (l.head_dim == 256 || sequences == 1)) return tiles;
-  // (a mean: each of several may well end on a page)
-  const uint32_t history = sequences > 1 ? committed - committed % KVX_PAGE_TOKENS : committed;
-  const auto shares = [&](uint32_t s) { return kvx_debug_prefill_by_chunk(layout, query_heads, history, rows, s); };
-  const auto time = [&](uint32_t s) { return prefill_chunk_time(l, history, rows, group, sequences, s); };
-  uint32_t best = 0;
-  double best_time = 0;
-  for (uint32_t s = 1; s <= most; ++s) {
-    if (!shares(s)) continue;
-    const double t = time(s);
-    if (best && t >= best_time) continue;
-    best = s;
-    best_time = t;
-  }
-  // the tiles' count stays where the estimate, 6 to 14 % off by itself, has less than a tenth against it
-  return !best || (shares(tiles) && best_time > 0.9 * time(tiles)) ? tiles : best;
 }
 int kvx_decode_plan_for(const kvx_layout *layout, const uint32_t *committed, uint32_t n_lanes,
                         uint32_t *split_counts) {

@@ -1,5 +1,6 @@
-"""kvx_prefill_plan_for where chunks run as workgroups of 256 fused rows: the split count is one that runs
-so, no split is shorter than 4 pages, and the sequences of a batch count as one launch."""
+"""kvx_prefill_plan_for is a function of the tiles: at head dimension 256 kvx_prefill_plan_batch's count, at 64 and
+128 the fewest splits that make 4096 workgroups of tiles.  Weights are rounded relative to the running maximum of
+the split they fall in, so a count that moves moves the rows of every engine that plans with it."""
 import ctypes as C
 
 import pytest
@@ -10,65 +11,54 @@ LAYOUTS = {"d256": (4, 6, 256), "d128": (2, 8, 128), "d64": (8, 4, 64)}
 FORMATS = {"int4": kvx.INT4, "int8": kvx.INT8, "fp8": kvx.FP8, "bf16": kvx.BF16}
 
 
+def layout_of(layout, fmt):
+    heads, _, dim = LAYOUTS[layout]
+    return kvx.Layout(1, heads, dim, FORMATS[fmt], 0.0)
+
+
 def plan(layout, fmt, committed, rows, sequences=1):
-    heads, group, dim = LAYOUTS[layout]
-    of = kvx.Layout(1, heads, dim, FORMATS[fmt], 0.0)
+    heads, group, _ = LAYOUTS[layout]
+    of = layout_of(layout, fmt)
     return kvx.lib().kvx_prefill_plan_for(C.byref(of), committed, rows, heads * group, sequences)
 
 
-def by_chunk(layout, fmt, committed, rows, splits):
-    heads, group, dim = LAYOUTS[layout]
-    of = kvx.Layout(1, heads, dim, FORMATS[fmt], 0.0)
-    return kvx.lib().kvx_debug_prefill_by_chunk(C.byref(of), heads * group, committed, rows, splits)
-
-
-@pytest.mark.parametrize("layout", sorted(LAYOUTS))
-@pytest.mark.parametrize("fmt", ("int8", "fp8", "bf16"))
-def test_the_planned_count_runs_as_workgroups_that_share_their_pages(layout, fmt):
-    for committed in (0, 32, 512, 1000, 4096, 16384, 100_000):
-        for rows in (64, 65, 255, 777, 2048):
-            for sequences in (1, 2, 3, 32):
-                splits = plan(layout, fmt, committed, rows, sequences)
-                assert 1 <= splits <= 32
-                mean = committed - committed % 32 if sequences > 1 else committed
-                possible = [s for s in range(1, 33) if by_chunk(layout, fmt, mean, rows, s)
-                            and (s == 1 or s * 4 <= (committed + rows // 2 + 31) // 32)]
-                if possible:
-                    assert by_chunk(layout, fmt, mean, rows, splits)
-
-
-def test_counts_of_full_rounds():
-    assert plan("d256", "bf16", 16384, 2048) == 4        # 192 workgroups a split: three full rounds of 256
-    assert plan("d256", "bf16", 16384, 2048, 4) == 1     # 768
-    assert plan("d256", "int8", 4032, 366, 2) == 3       # 72 a split
-    assert plan("d128", "fp8", 6144, 256, 2) == 16       # 32 a split: two rounds (8 splits would run tile by tile)
-    assert plan("d64", "bf16", 8192, 256) == 16          # 32 a split, 512 at a time
-    assert plan("d64", "int4", 288, 910, 4) == 2
-
-
 @pytest.mark.parametrize("fmt", sorted(FORMATS))
-def test_few_rows_at_head_dimension_256_keep_the_tiles_count_or_three(fmt):
-    for committed in (0, 100, 384, 4096, 65536):
-        for rows in (1, 33, 63):
-            old = kvx.prefill_plan(committed, rows, 4, 24, FORMATS[fmt])
-            pages = (committed + rows // 2 + 31) // 32
-            assert plan("d256", fmt, committed, rows) == max(old, min(3, max(1, pages // 4)))
+def test_head_dimension_256_is_the_batch_plan(fmt):
+    for committed in (0, 384, 1000, 4096, 16384, 100_000):
+        for rows in (1, 33, 40, 63, 64, 255, 777, 2048):
+            for sequences in (1, 2, 4, 16, 32):
+                want = kvx.prefill_plan(committed, rows, 4, 24, FORMATS[fmt], sequences)
+                assert plan("d256", fmt, committed, rows, sequences) == want
 
 
-def test_int4_alone_is_planned_by_tiles():
-    for committed, rows in ((0, 64), (384, 300), (16384, 2048)):
-        assert plan("d256", "int4", committed, rows) == kvx.prefill_plan(committed, rows, 4, 24, kvx.INT4)
-        for layout in ("d128", "d64"):  # the fewest splits that make 4096 workgroups of tiles, none below 4 pages
-            assert plan(layout, "int4", committed, rows) <= max(1, (committed + rows // 2 + 31) // 32 // 4)
+@pytest.mark.parametrize("fmt", ("bf16", "int8"))
+def test_batches_of_short_chunks_run_in_one_split(fmt):
+    # (63 bf16 rows of 32 sequences after 8256 tokens in three splits, tile by tile: 2490 us a layer for 575)
+    for rows in (33, 40, 63):
+        for sequences in (16, 32):
+            assert plan("d256", fmt, 8256, rows, sequences) == 1
 
 
-def test_sizes_beyond_the_limits_keep_the_tiles_count():
+@pytest.mark.parametrize("layout", ("d128", "d64"))
+@pytest.mark.parametrize("fmt", sorted(FORMATS))
+def test_head_dimensions_64_and_128_make_4096_workgroups_of_tiles(layout, fmt):
+    heads, group, _ = LAYOUTS[layout]
+    of = layout_of(layout, fmt)
+    for committed in (0, 288, 1000, 6144, 16384):
+        for rows in (33, 64, 256, 910, 2048):
+            most = min(32, max(1, (committed + rows // 2 + 31) // 32 // 4))
+            for splits in range(1, most + 1):
+                together = kvx.lib().kvx_debug_prefill_tiles_together(C.byref(of), heads * group, committed, rows, splits)
+                if -(-((rows + 7) // 8) // together) * heads * splits >= 4096:
+                    break
+            for sequences in (1, 2, 32):
+                assert plan(layout, fmt, committed, rows, sequences) == splits
+
+
+def test_sizes_beyond_the_limits_and_any_number_of_sequences():
     for committed, rows in ((0xFFFFFFFF, 64), (0, 0xFFFFFFFF), (0, 0), (1 << 20, 4096)):
         for layout in LAYOUTS:
             assert 0 <= plan(layout, "bf16", committed, rows) <= 32
-
-
-def test_any_number_of_sequences_is_planned():
     for sequences in (1000, 1 << 20, 0xFFFFFFFF):
         for layout in LAYOUTS:
             assert 1 <= plan(layout, "bf16", 16384, 2048, sequences) <= 32
