@@ -510,8 +510,8 @@ def tree_verify(args):
                      "mfma_frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4),
                      "kernel": ("verify32_int4_kernel (split kernel of verify attention, three waves of 32 fused rows)"
                                 if args.format == "int4" else
-                                "group_wide_kernel (split kernel of verify attention, four waves of 24 fused "
-                                "rows that share every page through LDS)") + ", one layer per launch",
+                                "verify_lane_kernel (split kernel of verify attention, waves of 32 fused rows "
+                                "beside waves that stage every page in LDS)") + ", one layer per launch",
                      "flops_per_launch": flops, "ms_per_launch": round(kernel_ms, 4),
                      "kv_gbs": round(kv_bytes / (kernel_ms * 1e-3) / 1e9, 1)},
         "cpu_baseline": None,
@@ -1173,8 +1173,8 @@ def chunked_prefill(args):
         "roofline": {"bound": "mfma", "achieved": round(achieved, 1), "peak": peak, "unit": "TFLOP/s",
                      "frac": round(achieved / peak, 4), "traffic": None,
                      "kernel": ("kv_attend_prefill_batch of one layer: every sequence's tiles in one launch of "
-                                "the split kernel (prefill_int4_kernel or chunk_attend_kernel)" if batched else
-                                "kv_attend_prefill of one sequence and layer: the split kernel (prefill_int4_kernel "
+                                "the split kernel (verify32_int4_kernel or chunk_attend_kernel)" if batched else
+                                "kv_attend_prefill of one sequence and layer: the split kernel (verify32_int4_kernel "
                                 "or chunk_attend_kernel) and, with several splits, the merge behind it"),
                      "flops_per_launch": flops, "ms_per_launch": round(kernel_ms, 4),
                      "sequences_per_launch": launch_sequences,

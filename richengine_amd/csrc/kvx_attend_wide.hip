@@ -580,8 +580,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES
 // pages; each wave keeps its quarter of one page in flight.  An operand read from LDS must
 // feed two row blocks: four waves reading one block's worth each would ask the LDS for
 // twice what it delivers.
-// (Verify lanes of more than 32 fused rows ran on it too, the forms with two waves, two register sets
-// or two copies below; they are verify_lane_kernel's now but for bf16 lanes of more than 96 rows.)
+// (Verify lanes of more than 32 fused rows are verify_lane_kernel's but for bf16 lanes of more than 96 rows.)
 constexpr uint32_t kGroupWaves = 4;
 
 // The workgroup's barrier between pairs of pages: a wave's LDS writes are done (the LDS
@@ -595,19 +594,18 @@ struct GroupOperands {
   u32x4 keys[2][8][64];  // [token block][dims block][lane]
   u32x4 values[16][64];  // [dims block][lane]
 };
-template <uint32_t FMT, uint32_t W>
-struct GroupShare {  // wave w's share of a page as loaded, W waves: dims blocks (8 / W) w .. of the
-                     // keys, dims blocks (16 / W) w .. of the values
-  static constexpr uint32_t kKeyBlocks = 8 / W, kValueBlocks = 16 / W;
+template <uint32_t FMT>
+struct GroupShare {  // wave w's share of a page as loaded: dims blocks 2 w .. of the keys, 4 w .. of the values
+  static constexpr uint32_t kKeyBlocks = 8 / kGroupWaves, kValueBlocks = 16 / kGroupWaves;
   uint32_t k[2][kKeyBlocks][Wide<FMT>::kDwords];  // [token block][dims block of the share]
   uint32_t v[kValueBlocks][Wide<FMT>::kDwords];
 };
 
-template <uint32_t FMT, uint32_t W, bool REUSED>
-__device__ __forceinline__ void fetch_share(GroupShare<FMT, W> &r, const PagePlace &p, uint32_t wave,
+template <uint32_t FMT, bool REUSED>
+__device__ __forceinline__ void fetch_share(GroupShare<FMT> &r, const PagePlace &p, uint32_t wave,
                                             uint32_t t, uint32_t g) {
   constexpr uint32_t B = Wide<FMT>::kBytes;
-  constexpr uint32_t KB = GroupShare<FMT, W>::kKeyBlocks, VB = GroupShare<FMT, W>::kValueBlocks;
+  constexpr uint32_t KB = GroupShare<FMT>::kKeyBlocks, VB = GroupShare<FMT>::kValueBlocks;
 #pragma unroll
   for (uint32_t tb = 0; tb < 2; ++tb) {
     const uint8_t *row = p.keys + (8 * (t >> 2) + 4 * tb + (t & 3)) * kD * B;
@@ -645,10 +643,10 @@ __device__ __forceinline__ u32x4 share_operand(const uint32_t (&raw)[Wide<FMT>::
   else if constexpr (Wide<FMT>::kInt8) return int8_operand(raw[0], raw[1]);
   else return u32x4{raw[0], raw[1], raw[2], raw[3]};
 }
-template <uint32_t FMT, uint32_t W>
-__device__ __forceinline__ void stage_share(GroupOperands &page, const GroupShare<FMT, W> &r, uint32_t wave,
+template <uint32_t FMT>
+__device__ __forceinline__ void stage_share(GroupOperands &page, const GroupShare<FMT> &r, uint32_t wave,
                                             uint32_t lane) {
-  constexpr uint32_t KB = GroupShare<FMT, W>::kKeyBlocks, VB = GroupShare<FMT, W>::kValueBlocks;
+  constexpr uint32_t KB = GroupShare<FMT>::kKeyBlocks, VB = GroupShare<FMT>::kValueBlocks;
 #pragma unroll
   for (uint32_t tb = 0; tb < 2; ++tb)
 #pragma unroll
@@ -657,21 +655,16 @@ __device__ __forceinline__ void stage_share(GroupOperands &page, const GroupShar
   for (uint32_t i = 0; i < VB; ++i) page.values[VB * wave + i][lane] = share_operand<FMT>(r.v[i]);
 }
 
-// NB blocks of 16 fused rows per wave; the lane's fused rows are dealt to the W waves in
-// equal runs of ceil(M / W) (at most 16 NB).  SETS register sets hold a wave's share of
-// the pages on their way: one, whose loads have a page time to arrive, for pages that come
-// out of the caches (prefill) and for bf16, whose share is 32 to 64 registers; two, with
-// two page times, for the byte formats' verify lanes, whose pages come from HBM.
-// COPIES staged pages in LDS: four (128 KiB, a barrier every second page) where the
-// workgroup's four waves fill the CU anyway; two (64 KiB, a barrier per page) for workgroups
-// of two waves, so that two of them fit a CU and no SIMD stays empty.
-template <uint32_t FMT, uint32_t NB, uint32_t W, bool REUSED, uint32_t SETS = 1, uint32_t COPIES = 4>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 1))) void
+// NB blocks of 16 fused rows per wave; the lane's fused rows are dealt to the four waves in
+// equal runs of ceil(M / 4) (at most 16 NB).  One register set holds a wave's share of a page on
+// its way, which has a page time to arrive; four staged pages in LDS (128 KiB, a barrier every
+// second page).
+template <uint32_t FMT, uint32_t NB, bool REUSED>
+__global__ __launch_bounds__(64 * kGroupWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
                   float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
   constexpr bool kFp8 = Wide<FMT>::kFp8, kInt8 = Wide<FMT>::kInt8, kByte = Wide<FMT>::kByte;
-  static_assert(COPIES == 4 || (COPIES == 2 && SETS == 1), "two copies: one set of page registers");
-  __shared__ GroupOperands shared_page[COPIES];
+  __shared__ GroupOperands shared_page[4];
   const uint32_t item = blockIdx.x, head = blockIdx.y;
   uint32_t li;
   const DecodeLane l = lane_of_item(a, item, li);
@@ -694,7 +687,7 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
   const RegionOffsets ro = region_offsets(a.kv.extent_pages, db, sb);
   const float score_scale = default_score_scale(kD, l.score_scale);
 
-  const uint32_t run = (M + W - 1) / W;  // fused rows per wave
+  const uint32_t run = (M + kGroupWaves - 1) / kGroupWaves;  // fused rows per wave
   uint32_t m[NB];
   bool in_tile[NB], live_row[NB];
   Sight sight[NB];
@@ -737,8 +730,7 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
 
   const uint64_t *const entries = l.table + begin;
   const uint32_t count = end - begin, last_slot = count - 1;
-  static_assert(SETS == 1 || (SETS == 2 && Wide<FMT>::kByte), "two sets of page registers: byte formats only");
-  GroupShare<FMT, W> raw[SETS];  // this wave's share of the pages on their way
+  GroupShare<FMT> raw;  // this wave's share of the page on its way
   // bf16 pages: a page's entry is read a turn before the loads that need it, since one wave
   // per SIMD has nothing else to run while a scalar load is on its way.  With the byte
   // formats' conversions to fill that time the early read measured 10 % slower, and they
@@ -750,10 +742,10 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
     entry_ahead = scalar_entry(entries, min(following, last_slot));
     return entry;
   };
-  auto fetch = [&](GroupShare<FMT, W> &set, uint64_t entry) {
+  auto fetch = [&](uint64_t entry) {
     const PagePlace p = place_page<FMT>(entry, head, H, a.kv.offset, ro);
     asm volatile("");
-    fetch_share<FMT, W, REUSED>(set, p, wave, t, g);
+    fetch_share<FMT, REUSED>(raw, p, wave, t, g);
     asm volatile("");
   };
   // The scales of a byte format's page, by every wave for its own lanes: they are few, and
@@ -768,43 +760,8 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
       vs[1] = load_global<f32x4>(p.value_scales + 8 * g + 4);
     }
   };
-  // bf16 pages need no conversion on their way: in the two-copy form the wave's share of a
-  // page goes from global memory into the staged copy directly (16 bytes per lane and
-  // instruction, the lanes of an instruction one operand block), with no registers in between
-  // and no LDS writes to issue.  The copy must be free when the loads are sent, since they
-  // land whenever they arrive; the wave waits for them before the barrier that hands the copy
-  // over.  (bf16 chain verify of a batch of 32: 413 -> 396 us.  The four-copy form was slower
-  // with it, a 2048-row prefill chunk 1.19 -> 1.27 ms, and stages through registers.)
-  constexpr bool kDirect = !kByte && COPIES == 2;
-  auto direct = [&](GroupOperands &copy, uint64_t entry) {
-    constexpr uint32_t B = Wide<FMT>::kBytes;
-    constexpr uint32_t KB = GroupShare<FMT, W>::kKeyBlocks, VB = GroupShare<FMT, W>::kValueBlocks;
-    constexpr uint32_t kPolicy = REUSED ? 0u : 2u;  // 2: non-temporal, for pages read once
-    typedef __attribute__((address_space(1))) const void GlobalBytes;
-    typedef __attribute__((address_space(3))) void SharedBytes;
-    const PagePlace p = place_page<FMT>(entry, head, H, a.kv.offset, ro);
-#pragma unroll
-    for (uint32_t tb = 0; tb < 2; ++tb) {
-      const uint8_t *row = p.keys + (8 * (t >> 2) + 4 * tb + (t & 3)) * kD * B;
-#pragma unroll
-      for (uint32_t c = 0; c < KB; ++c)
-        __builtin_amdgcn_global_load_lds(
-            (GlobalBytes *)(reinterpret_cast<uintptr_t>(row + key_dims<FMT>(KB * wave + c, g) * B)),
-            (SharedBytes *)(&copy.keys[tb][KB * wave + c][0]), 16, 0, kPolicy);
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < VB; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (GlobalBytes *)(reinterpret_cast<uintptr_t>(p.values + ((16 * (VB * wave + i) + t) * kPage + 8 * g) * B)),
-          (SharedBytes *)(&copy.values[VB * wave + i][0]), 16, 0, kPolicy);
-  };
-  // The barrier of the direct form: the wave's loads into the copies have landed.
-  auto landed_barrier = [&] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   const uint64_t entry0 = next_entry(1), entry1 = next_entry(2);
-  if constexpr (!kDirect) {
-    fetch(raw[0], entry0);
-    if constexpr (SETS == 2) fetch(raw[1], entry1);
-  }
+  fetch(entry0);
   fetch_scales(ks_even, vs_even, entry0);
   fetch_scales(ks_odd, vs_odd, entry1);
 
@@ -925,87 +882,41 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
   };
 
   const uint32_t first_masked = l.committed / kPage;
-  if constexpr (kDirect) {
-    // Two copies, loaded directly: while slot i is multiplied out of one, slot i + 1 lands in
-    // the other; a barrier per page.
-    direct(shared_page[0], entry0);
-    landed_barrier();
-    auto turn = [&](const GroupOperands &now, GroupOperands &next, uint32_t slot) __attribute__((always_inline)) {
-      direct(next, slot == 0 ? entry1 : next_entry(slot + 2));  // of slot + 1
-      if (computes && slot < count) attend_page(now, begin + slot, ks_even, vs_even, begin + slot >= first_masked);
-      landed_barrier();
-    };
-    for (uint32_t slot = 0; slot < count; slot += 2) {
-      turn(shared_page[0], shared_page[1], slot);
-      turn(shared_page[1], shared_page[0], slot + 1);
-    }
-  } else if constexpr (COPIES == 2) {
-    // Two copies: while slot i is multiplied out of one, slot i + 1 goes from the raw
-    // registers into the other and the registers are sent for slot i + 2; a barrier per page.
-    stage_share<FMT, W>(shared_page[0], raw[0], wave, lane);
-    fetch(raw[0], entry1);
+  // The first two pages into the first two copies; held: the entry of the page whose operands are on
+  // their way (slot + 2 of a pair), whose scales are asked for a page time later.
+  stage_share<FMT>(shared_page[0], raw, wave, lane);
+  fetch(entry1);
+  stage_share<FMT>(shared_page[1], raw, wave, lane);
+  uint64_t held = next_entry(3);
+  fetch(held);
+  group_barrier();
+  // Four copies, two pages between barriers: while slots i and i + 1 are multiplied out of
+  // one pair of copies, slots i + 2 and i + 3 go from the raw registers into the other pair,
+  // each one page time after its loads were sent (past the end: the last page again, staged into
+  // copies nobody reads).  A barrier per page cost 5 % more: the waves leave it together and read
+  // their operands at the same time.  Four slots per turn of the loop and no branch around the
+  // loads, so every wait names exactly the loads it needs.
+  auto pair = [&](const GroupOperands &now0, const GroupOperands &now1, GroupOperands &next0,
+                  GroupOperands &next1, uint32_t slot) __attribute__((always_inline)) {
+    stage_share<FMT>(next0, raw, wave, lane);  // slot + 2
+    const uint64_t entry_a = next_entry(slot + 4);  // of slot + 3
+    fetch(entry_a);
+    if (computes && slot < count)
+      attend_page(now0, begin + slot, ks_even, vs_even, begin + slot >= first_masked);
+    fetch_scales(ks_even, vs_even, held);  // of slot + 2
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    stage_share<FMT>(next1, raw, wave, lane);  // slot + 3
+    const uint64_t entry_b = next_entry(slot + 5);  // of slot + 4
+    fetch(entry_b);
+    if (computes && slot + 1 < count)
+      attend_page(now1, begin + slot + 1, ks_odd, vs_odd, begin + slot + 1 >= first_masked);
+    fetch_scales(ks_odd, vs_odd, entry_a);  // of slot + 3
+    held = entry_b;
     group_barrier();
-    auto turn = [&](const GroupOperands &now, GroupOperands &next, uint32_t slot, f32x4 (&ks)[2],
-                    f32x4 (&vs)[2]) __attribute__((always_inline)) {
-      stage_share<FMT, W>(next, raw[0], wave, lane);  // slot + 1
-      const uint64_t entry = next_entry(slot + 3);  // of slot + 2
-      fetch(raw[0], entry);
-      if (computes && slot < count) attend_page(now, begin + slot, ks, vs, begin + slot >= first_masked);
-      fetch_scales(ks, vs, entry);
-      group_barrier();
-    };
-    for (uint32_t slot = 0; slot < count; slot += 2) {
-      turn(shared_page[0], shared_page[1], slot, ks_even, vs_even);
-      turn(shared_page[1], shared_page[0], slot + 1, ks_odd, vs_odd);
-    }
-  } else {
-    // The first two pages into the first two copies; the entries of the pages whose operands are on their way (slots + 2 and + 3 of a pair):
-    // their scales are asked for a page time later.
-    uint64_t held_even, held_odd = 0;
-    stage_share<FMT, W>(shared_page[0], raw[0], wave, lane);
-    if constexpr (SETS == 1) {
-      fetch(raw[0], entry1);
-      stage_share<FMT, W>(shared_page[1], raw[0], wave, lane);
-      held_even = next_entry(3);
-      fetch(raw[0], held_even);
-    } else {
-      held_even = next_entry(3);
-      fetch(raw[0], held_even);
-      stage_share<FMT, W>(shared_page[1], raw[1], wave, lane);
-      held_odd = next_entry(4);
-      fetch(raw[1], held_odd);
-    }
-    group_barrier();
-    // Four copies, two pages between barriers: while slots i and i + 1 are multiplied out of
-    // one pair of copies, slots i + 2 and i + 3 go from the raw registers into the other pair,
-    // each one page time (two with two sets) after its loads were sent (past the end: the last
-    // page again, staged into copies nobody reads).  A barrier per page cost 5 % more: the
-    // waves leave it together and read their operands at the same time.  Four slots per turn
-    // of the loop and no branch around the loads, so every wait names exactly the loads it
-    // needs.
-    auto pair = [&](const GroupOperands &now0, const GroupOperands &now1, GroupOperands &next0,
-                    GroupOperands &next1, uint32_t slot) __attribute__((always_inline)) {
-      stage_share<FMT, W>(next0, raw[0], wave, lane);  // slot + 2
-      const uint64_t entry_a = next_entry(slot + 3 + SETS);  // of slot + 2 + SETS
-      fetch(raw[0], entry_a);
-      if (computes && slot < count)
-        attend_page(now0, begin + slot, ks_even, vs_even, begin + slot >= first_masked);
-      fetch_scales(ks_even, vs_even, held_even);  // of slot + 2
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      stage_share<FMT, W>(next1, raw[SETS - 1], wave, lane);  // slot + 3
-      const uint64_t entry_b = next_entry(slot + 4 + SETS);  // of slot + 3 + SETS
-      fetch(raw[SETS - 1], entry_b);
-      if (computes && slot + 1 < count)
-        attend_page(now1, begin + slot + 1, ks_odd, vs_odd, begin + slot + 1 >= first_masked);
-      fetch_scales(ks_odd, vs_odd, SETS == 1 ? entry_a : held_odd);  // of slot + 3
-      held_even = SETS == 1 ? entry_b : entry_a;
-      held_odd = entry_b;
-      group_barrier();
-    };
-    for (uint32_t slot = 0; slot < count; slot += 4) {
-      pair(shared_page[0], shared_page[1], shared_page[2], shared_page[3], slot);
-      pair(shared_page[2], shared_page[3], shared_page[0], shared_page[1], slot + 2);
-    }
+  };
+  for (uint32_t slot = 0; slot < count; slot += 4) {
+    pair(shared_page[0], shared_page[1], shared_page[2], shared_page[3], slot);
+    pair(shared_page[2], shared_page[3], shared_page[0], shared_page[1], slot + 2);
   }
   if (!computes) return;
 
@@ -1050,19 +961,6 @@ group_wide_kernel(const uint16_t *__restrict__ queries, uint16_t *__restrict__ o
   }
 }
 
-// No launch takes these forms any more; tests/test_abi.py still holds the registers and scratch memory they
-// compile to.
-#define KVX_HELD(...)                                                                                  \
-  template __global__ void group_wide_kernel<__VA_ARGS__>(const uint16_t *__restrict__, uint16_t *__restrict__, \
-                                                          float *__restrict__, float *__restrict__, DecodeArgs);
-KVX_HELD(KVX_FMT_INT8, 2, 4, false, 2)
-KVX_HELD(KVX_FMT_FP8E4M3, 2, 4, false, 2)
-KVX_HELD(KVX_FMT_INT8, 2, 2, false, 1, 2)
-KVX_HELD(KVX_FMT_FP8E4M3, 2, 2, false, 1, 2)
-KVX_HELD(KVX_FMT_BF16, 2, 2, false, 1, 2)
-KVX_HELD(KVX_FMT_BF16, 3, 2, false, 1, 2)
-#undef KVX_HELD
-
 }  // namespace
 }  // namespace kvx
 
@@ -1106,21 +1004,21 @@ int kvx_attend_wide_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
   // The regular tiles of a chunked prefill (tile_rows > 0) walk the same pages
   // over and over: their loads may stay in the caches.
   const bool reused = tile_rows > 0;
-#define KVX_GROUP(FMT, NB, W, REUSED, ...)                                                        \
-  launch_matrix_attention(group_wide_kernel<FMT, NB, W, REUSED, ##__VA_ARGS__>, "group_wide_kernel", 16 * NB * W, 64 * W, \
-                          s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, row_masks, \
-                          row_stride, lane_stride, workspace, workspace_bytes, stream, nullptr,     \
+#define KVX_GROUP(FMT, NB, REUSED)                                                                 \
+  launch_matrix_attention(group_wide_kernel<FMT, NB, REUSED>, "group_wide_kernel", 16 * NB * kGroupWaves, \
+                          64 * kGroupWaves, s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, \
+                          row_masks, row_stride, lane_stride, workspace, workspace_bytes, stream, nullptr, \
                           tile_rows, epilogue)
-#define KVX_GROUP_FORMATS(NB, W, REUSED)                                                          \
-  (format == KVX_FMT_BF16   ? KVX_GROUP(KVX_FMT_BF16, NB, W, REUSED)                                \
-   : format == KVX_FMT_INT8 ? KVX_GROUP(KVX_FMT_INT8, NB, W, REUSED)                                \
-                            : KVX_GROUP(KVX_FMT_FP8E4M3, NB, W, REUSED))
+#define KVX_GROUP_FORMATS(NB)                                                                      \
+  (format == KVX_FMT_BF16   ? KVX_GROUP(KVX_FMT_BF16, NB, true)                                      \
+   : format == KVX_FMT_INT8 ? KVX_GROUP(KVX_FMT_INT8, NB, true)                                      \
+                            : KVX_GROUP(KVX_FMT_FP8E4M3, NB, true))
   // many_tiles == 2: lanes of several prefill tiles each, for a workgroup of four waves
   // that shares every page through LDS, two or three row blocks per wave: up to 192 fused rows.
   if (many_tiles == 2) {
     if (!tile_rows || M > 48u * kGroupWaves) return 1;
-    if (M > 32u * kGroupWaves) return KVX_GROUP_FORMATS(3, 4, true);
-    return KVX_GROUP_FORMATS(2, 4, true);
+    if (M > 32u * kGroupWaves) return KVX_GROUP_FORMATS(3);
+    return KVX_GROUP_FORMATS(2);
   }
   // Verify lanes of more than 32 fused rows, which hold 128 at most, and the rows of sequences over a prefix they
   // share: waves that multiply beside waves that stage.  (Few workgroups are as fast, 16 lanes of 1200 tokens at
@@ -1131,7 +1029,7 @@ int kvx_attend_wide_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
     if (format != KVX_FMT_BF16 || M <= 96 || shared_prefix)
       return kvx_verify_lane_launch(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, row_masks,
                                     row_stride, lane_stride, workspace, workspace_bytes, stream, epilogue);
-    return KVX_GROUP(KVX_FMT_BF16, 2, 4, false);
+    return KVX_GROUP(KVX_FMT_BF16, 2, false);
   }
 #undef KVX_GROUP_FORMATS
 #undef KVX_GROUP

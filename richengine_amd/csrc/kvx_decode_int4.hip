@@ -856,6 +856,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
   attend_int4<2, 1, true, false, true>(queries, output, partials, statistics, a);
 }
+
 // Single tiles of a chunked prefill, and pairs of no more than 16 fused rows: a wave to a workgroup with
 // two register sets of pages (as waves of verify_int4_kernel 256 rows after 8192 tokens in five splits
 // took 168 us instead of 133, one tile after 40 000 in sixteen 143 instead of 99).
@@ -863,12 +864,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
     float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
   attend_int4<1, kDecodeDepth, true>(queries, output, partials, statistics, a);
-}
-// Pairs of tiles in waves of 32 rows: verify32_int4_kernel under a name of its own in a trace.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_int4_kernel(
-    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
-    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
-  attend_int4<2, 1, true, false, true>(queries, output, partials, statistics, a);
 }
 
 // Three blocks (48 fused rows: a chain of 8 rows for a group of 6 query heads) read and expand every
@@ -989,7 +984,7 @@ int kvx_attend_int4_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
                                      query_heads, queries, output, page_tables, lanes, n_lanes,
                                      row_masks, row_stride, lane_stride, workspace, workspace_bytes,
                                      stream, nullptr, tile_rows, epilogue);
-    return launch_matrix_attention(rows == 16 ? verify_int4_kernel : tile_rows ? prefill_int4_kernel : verify32_int4_kernel,
+    return launch_matrix_attention(rows == 16 ? verify_int4_kernel : verify32_int4_kernel,
                                    "int4 kernels of several row blocks", rows, 256, s, kv, query_heads,
                                    queries, output, page_tables, lanes, n_lanes, row_masks, row_stride,
                                    lane_stride, workspace, workspace_bytes, stream, nullptr, tile_rows,

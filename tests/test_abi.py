@@ -302,12 +302,12 @@ def test_decode_and_verify_plans_size_the_launch_for_the_gpu():
 
 def test_hot_kernels_stay_out_of_scratch_memory():
     """What the compiler reported when the library was built (written next to it by
-    richengine_amd/build.py): the kernels of the decode path and the verify kernel must
-    not touch scratch memory -- a spill reload or an argument block moved to scratch waits
-    behind every page load in flight -- and the int4 decode kernel must fit two waves per
-    SIMD."""
+    richengine_amd/build.py): the kernels of the decode and verify paths must not touch
+    scratch memory -- a spill reload or an argument block moved to scratch waits behind every
+    page load in flight -- and must fit the waves per SIMD that they are launched for."""
     import json
     import os
+    import re
     from richengine_amd import build as kvx_build
     if not os.path.exists(kvx_build.RESOURCES):
         pytest.skip("the library was built without the compiler's resource report")
@@ -319,7 +319,7 @@ def test_hot_kernels_stay_out_of_scratch_memory():
         return report[names[0]]
 
     for fragment in ("decode_int4_kernelE", "decode_int4_quad_kernel", "decode_int4_tiles_kernel", "verify_int4_kernel",
-                     "verify32_int4_kernel", "verify48_int4_kernel", "prefill_int4_kernel",
+                     "verify32_int4_kernel", "verify48_int4_kernel",
                      "matrix_merge_kernelILj1E", "matrix_merge_kernelILj8E",   # one wave per row; ranged
                      "attend_wide_kernelILj1ELj1ELj2ELb0E",    # int8, one block, two waves per SIMD
                      "attend_wide_kernelILj4ELj1ELj2ELb0E",    # fp8
@@ -333,26 +333,36 @@ def test_hot_kernels_stay_out_of_scratch_memory():
         assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, (fragment, r)
     assert one("decode_int4_kernelE")["occupancy"] == 2 and one("decode_int4_quad_kernel")["occupancy"] == 2
     # two blocks over one page set: every accumulator in the first register file
-    assert one("verify32_int4_kernel")["agprs"] == 0 and one("prefill_int4_kernel")["agprs"] == 0
+    assert one("verify32_int4_kernel")["agprs"] == 0
+    # waves of 16 rows: three to a SIMD
+    assert one("verify_int4_kernel")["occupancy"] == 3
     # the workgroup-shared prefill kernels (int8, bf16, fp8 pages; two and three row blocks
     # per wave): one wave per SIMD with all 512 registers; the byte formats' three-block forms
     # park a few set-up values in scratch memory, none of them touched inside the page loop
     # (no scratch access in the loop's assembly when this bound was set)
-    # (the same kernels with loads that do not stay in the caches serve tree verify, and forms
-    # with two waves and two LDS copies a chain of 8 rows)
+    # (the two-block bf16 form with loads that do not stay in the caches serves verify lanes of more
+    # than 96 rows)
     for fmt in (1, 2, 4):
         for blocks in (2, 3):
-            for reused in ((0, 1) if blocks == 2 else (1,)):
-                r = one(f"group_wide_kernelILj{fmt}ELj{blocks}ELj4ELb{reused}E")
-                if fmt != 2 and blocks == 3:
-                    assert r["vgprs_spill"] <= 10, (fmt, blocks, r)
-                else:
-                    assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, (fmt, blocks, r)
-    for fmt in (1, 2, 4):
-        r = one(f"group_wide_kernelILj{fmt}ELj2ELj2ELb0E")
-        assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, r
-    r = one("group_wide_kernelILj2ELj3ELj2ELb0E")      # bf16, two waves of 48 rows, direct loads
+            r = one(f"group_wide_kernelILj{fmt}ELj{blocks}ELb1E")
+            if fmt != 2 and blocks == 3:
+                assert r["vgprs_spill"] <= 10, (fmt, blocks, r)
+            else:
+                assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, (fmt, blocks, r)
+    r = one("group_wide_kernelILj2ELj2ELb0E")
     assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, r
+    # verify lanes of 33 to 128 rows and shared prefixes, one-row decode at head dimensions 64 and 128: every
+    # form, at the waves a SIMD that it is built for
+    lanes = [n for n in report if "verify_lane_kernelI" in n]
+    assert len(lanes) == 7
+    for name in lanes:
+        r = report[name]
+        assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0 and r["occupancy"] == 2, (name, r)
+    small = [n for n in report if "decode_small_kernelI" in n]
+    assert len(small) == 9
+    for name in small:
+        r, waves = report[name], int(re.search(r"ELj(\d)EEEv", name).group(1))
+        assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0 and r["occupancy"] == waves, (name, r)
     # head dimensions 64 and 128, a wave per tile: no scratch, and two (128) or three and more
     # (64) waves per SIMD beside the staged copies
     for fmt in (1, 2, 3, 4):
