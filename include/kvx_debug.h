@@ -28,6 +28,11 @@ uint32_t kvx_debug_prefill_by_chunk(const kvx_layout *layout, uint32_t query_hea
 uint32_t kvx_debug_prefill_tiles_together(const kvx_layout *layout, uint32_t query_heads,
                                           uint32_t committed_tokens, uint32_t rows, uint32_t splits);
 
+/* Fused query rows to a wave (16, 32 or 48) of a kv_attend_verify call of these lanes on int4 pages of head
+   dimension 256 (0: invalid arguments or other pages), so tests can tell which kernel a lane ran on. */
+uint32_t kvx_debug_int4_verify_rows(const kvx_layout *layout, uint32_t query_heads,
+                                    const kvx_verify_params *lanes, uint32_t n_lanes);
+
 /* Streams the pages of `page_table` (n_pages device entries of an int4, head dimension 256
    storage) with exactly the loads of the int4 decode kernel, two waves per SIMD, and nothing
    behind them; workgroup x reads entries x * pages_per_wave onward, one wave per KV head,

@@ -948,6 +948,17 @@ static uint32_t int4_blocks(uint32_t kv_heads, uint32_t fused_rows, const kvx_ve
   return waves <= 3072 ? 16 : 32;
 }
 
+extern "C" uint32_t kvx_debug_int4_verify_rows(const kvx_layout *layout, uint32_t query_heads,
+                                               const kvx_verify_params *lanes, uint32_t n_lanes) {
+  if (!kvx_layout_valid(layout) || layout->format != KVX_FMT_INT4 || layout->head_dim != kD || !query_heads ||
+      query_heads % layout->kv_heads || !lanes || !n_lanes)
+    return 0;
+  const uint32_t fused_rows = lanes[0].row_capacity * (query_heads / layout->kv_heads);
+  for (uint32_t i = 0; i < n_lanes; ++i)
+    if (!lanes[i].split_count) return 0;
+  return fused_rows <= 16 ? 16 : int4_blocks(layout->kv_heads, fused_rows, lanes, n_lanes, false);
+}
+
 // Runs paged attention (split kernel, then the merge of multi-split lanes) for
 // int4 pages of head dimension 256; returns 1 (declined) for shapes it does not
 // cover so the caller runs the format-generic kernels, 0 when enqueued, or a

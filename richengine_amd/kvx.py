@@ -36,7 +36,7 @@ SYMBOLS = [
     "kvx_pool_free_pages", "kvx_pool_reclaim_empty", "kvx_pool_compact_extent",
     "kvx_pool_snapshot_get", "kv_append", "kv_prepare_append", "kv_attend_decode_shared", "kvx_attend_shared_workspace_bytes", "kv_attend_verify", "kv_attend_verify_hidden", "kv_attend_decode",
     "kv_attend_prefill", "kv_attend_prefill_batch", "kv_compact_path", "kv_append_attend_decode", "kv_append_attend_decode_hidden", "kv_page_export", "kv_page_import", "kv_attend_split", "kv_attend_merge", "kv_attend_decode_static",
-    "kvx_debug_attend_paths", "kvx_debug_prefill_tiles_together", "kvx_debug_prefill_by_chunk", "kvx_calibrate_stream", "kvx_decode_plan", "kvx_decode_plan_for", "kvx_prefill_plan_for", "kvx_verify_plan", "kvx_storage_create_accounting", "kvx_prefix_create", "kvx_prefix_destroy", "kvx_prefix_find",
+    "kvx_debug_attend_paths", "kvx_debug_prefill_tiles_together", "kvx_debug_prefill_by_chunk", "kvx_debug_int4_verify_rows", "kvx_calibrate_stream", "kvx_decode_plan", "kvx_decode_plan_for", "kvx_prefill_plan_for", "kvx_verify_plan", "kvx_storage_create_accounting", "kvx_prefix_create", "kvx_prefix_destroy", "kvx_prefix_find",
     "kvx_prefix_insert", "kvx_prefix_contains", "kvx_prefix_generation", "kvx_prefix_block_count",
     "kvx_prefix_chain", "kvx_prefix_retain_active", "kvx_prefix_release_active",
     "kvx_prefix_touch", "kvx_prefix_eviction_candidate", "kvx_prefix_erase",
@@ -202,6 +202,7 @@ def _declare(L):
     L.kvx_debug_prefill_tiles_together.restype = u32
     L.kvx_debug_prefill_by_chunk.argtypes = [LP, u32, u32, u32, u32]
     L.kvx_debug_prefill_by_chunk.restype = u32
+    L.kvx_debug_int4_verify_rows.argtypes, L.kvx_debug_int4_verify_rows.restype = [LP, u32, vp, u32], u32
     L.kvx_calibrate_stream.argtypes = [vp, u32, vp, u32, u32, u32, vp, vp]
     L.kvx_calibrate_stream_form.argtypes = [vp, u32, vp, u32, u32, u32, u32, u32, vp, vp]
     L.kvx_decode_plan.argtypes = [vp, u32, u32, u32, vp]
