@@ -18,6 +18,8 @@ hundred tokens (a seeded search over random shapes: int8 pages, a prefix of one 
 the oracle's two arrangements lay exactly as far apart as the library's).  So the library is
 held to the oracle's own distance between the two arrangements, row by row, plus the bar.
 """
+import sys
+
 import numpy as np
 import pytest
 
@@ -71,13 +73,30 @@ def shared_pool(fmt, shared_pages, own_tokens, seed, layer=1):
     return tw, hts, dts, [shared_pages + n for n in own_pages]
 
 
+@pytest.fixture
+def group(request, monkeypatch):
+    """(KV heads, group) in place of 4 x 6 for this file's helpers."""
+    monkeypatch.setattr(sys.modules[__name__], "H", request.param[0])
+    monkeypatch.setattr(sys.modules[__name__], "G", request.param[1])
+    monkeypatch.setattr(sys.modules[__name__], "QH", request.param[0] * request.param[1])
+    return request.param
+
+
 @pytest.mark.parametrize("fmt", [ko.INT4, ko.INT8, ko.BF16])
-@pytest.mark.parametrize("shared_pages,own_tokens,prefix_splits", [
-    (40, [0, 5, 31, 32, 700, 64, 1], 5),      # 7 sequences: 42 fused rows over the prefix
-    (3, [10, 2000], 1),                      # 12 fused rows: the one-block kernel; a single prefix split
-    (129, [3] * 16, 16),                     # 16 sequences, 96 fused rows
-])
-def test_shared_prefix_decode_matches_oracle(fmt, shared_pages, own_tokens, prefix_splits):
+@pytest.mark.parametrize("group,shared_pages,own_tokens,prefix_splits,row_stride", [
+    ((4, 6), 40, [0, 5, 31, 32, 700, 64, 1], 5, 1),  # 7 sequences: 42 fused rows over the prefix
+    ((4, 6), 3, [10, 2000], 1, 1),                   # 12 fused rows: the one-block kernel; a single prefix split
+    ((4, 6), 129, [3] * 16, 16, 1),                  # 16 sequences, 96 fused rows
+    # queries and output with rows between the heads' (12, 24, 42 fused rows), the heads' rows far apart
+    ((4, 6), 7, [40, 3], 2, 32),
+    ((3, 8), 33, [0, 17, 90], 4, 32),
+    ((2, 6), 12, [0, 5, 31, 32, 70, 64, 1], 3, 5),
+    ((2, 14), 20, [9, 0, 33, 64, 1, 2, 3], 6, 2),    # 98 fused rows: two in the fourth wave of 32
+    ((1, 16), 9, [31, 70, 0, 5, 6, 7, 8, 9], 2, 1),  # 128
+    ((2, 8), 17, [1 + i for i in range(16)], 3, 32),  # 128, sixteen sequences
+    ((3, 1), 8, [5, 45], 1, 4),                      # two fused rows
+], indirect=["group"])
+def test_shared_prefix_decode_matches_oracle(fmt, group, shared_pages, own_tokens, prefix_splits, row_stride):
     import torch
     import gpulib as Gp
     import test_gpu_attention as A
@@ -85,6 +104,9 @@ def test_shared_prefix_decode_matches_oracle(fmt, shared_pages, own_tokens, pref
     tw, hts, dts, entries = shared_pool(fmt, shared_pages, own_tokens, seed=300 + shared_pages)
     committed = [shared_pages * 32 + t for t in own_tokens]
     q = A.queries((lanes, H, 1, G, D), 17)
+    strided = np.zeros((lanes, H, row_stride, G, D), dtype=np.uint16)
+    strided[:, :, :1] = q
+    given = Gp.dev(strided)
     want = np.zeros((lanes, H, G, D), dtype=np.uint16)
     want32 = np.zeros((lanes, H, G, D), dtype=np.float32)
     for i in range(lanes):
@@ -100,13 +122,14 @@ def test_shared_prefix_decode_matches_oracle(fmt, shared_pages, own_tokens, pref
           for i in range(lanes)]
     ws = torch.empty(kvx.attend_shared_workspace_bytes(tw.dev, dp, prefix_splits, QH), dtype=torch.uint8,
                      device="cuda")
-    out = torch.full((lanes, H, 1, G, D), 0x5A5A, dtype=torch.int16, device="cuda")
-    kvx.attend_decode_shared(tw.dev, 1, QH, Gp.dev(q), out, dts, dp, shared_pages, prefix_splits, 1, ws)
+    out = torch.full((lanes, H, row_stride, G, D), 0x5A5A, dtype=torch.int16, device="cuda")
+    kvx.attend_decode_shared(tw.dev, 1, QH, given, out, dts, dp, shared_pages, prefix_splits, row_stride, ws)
     torch.cuda.synchronize()
+    assert (Gp.host_u16(out)[:, :, 1:] == 0x5A5A).all()
     got = Gp.host_u16(out)[:, :, 0]
     same, same32 = oracle_shared(fmt, tw, hts, entries, q, shared_pages, own_tokens, prefix_splits, own_splits)
     Gp.check_attention(got, same, same32, np.ones((lanes, H), dtype=bool), A.tol(fmt),
-                       f"shared prefix fmt={fmt} pages={shared_pages}",
+                       f"shared prefix fmt={fmt} group={group} pages={shared_pages}",
                        explain=lambda index: dict(rows=flipped_rows(
                            fmt, tw, hts, entries, q, shared_pages, own_tokens, prefix_splits, own_splits,
                            committed, index)))
@@ -121,15 +144,15 @@ def test_shared_prefix_decode_matches_oracle(fmt, shared_pages, own_tokens, pref
     up = [kvx.VerifyParams(committed[i], entries[i], kvx.KvLayer(), kvx.lib().kvx_decode_splits(committed[i], 1),
                            128, 1, 1, 0.0) for i in range(lanes)]
     ws2 = torch.empty(kvx.attend_workspace_bytes(tw.dev, up, QH), dtype=torch.uint8, device="cuda")
-    kvx.attend_decode(tw.dev, 1, QH, Gp.dev(q), plain, dts, up, 1, ws2)
+    kvx.attend_decode(tw.dev, 1, QH, given, plain, dts, up, row_stride, ws2)
     torch.cuda.synchronize()
     a = ko.bf16_to_f32(got).reshape(got.shape).astype(np.float64)
     b = ko.bf16_to_f32(Gp.host_u16(plain)[:, :, 0]).reshape(got.shape).astype(np.float64)
     relative = np.linalg.norm(a - b, axis=-1) / np.linalg.norm(b, axis=-1)
     assert (relative <= between + 2 * A.tol(fmt)).all(), (relative.max(), between.max())
     # the same call again gives the same bits
-    again = torch.zeros_like(out)
-    kvx.attend_decode_shared(tw.dev, 1, QH, Gp.dev(q), again, dts, dp, shared_pages, prefix_splits, 1, ws)
+    again = torch.full_like(out, 0x5A5A)
+    kvx.attend_decode_shared(tw.dev, 1, QH, given, again, dts, dp, shared_pages, prefix_splits, row_stride, ws)
     torch.cuda.synchronize()
     assert torch.equal(out, again)
     tw.close()
