@@ -369,14 +369,14 @@ int kvx_decode_plan_for(const kvx_layout *layout, const uint32_t *committed, uin
   for (uint32_t i = 0; i < n_lanes; ++i)
     if (uint64_t(committed[i]) + 1 > KVX_MAX_PHYSICAL_TOKENS)
       return fail(KVX_EINVAL, "kvx_decode_plan_for: context_out_of_range");
-  // Head dimensions 64 and 128: a wave per (lane, KV head, split) over a staged copy of the
-  // page's values of its own, sixteen waves to a CU (eight at head dimension 128 over pages
-  // other than int4, whose raw bytes take more registers); one round of them, splits of at
-  // least 4 pages (32 sequences of 8192 tokens, int4, 2 x 8 x 128: 48 us at 64 splits, 51 at
-  // 32, 60 at 128; 8 x 4 x 64: 83 us at 16, 82 at 32, 85 at 64; int8 2 x 8 x 128: 44 us at 32,
-  // 49 at 64).  bf16 pages are read at close to the memory's rate with half as many waves, and
-  // the other half only adds partial rows (2 x 8 x 128: 54 us at 16 splits, 55 at 32; 8 x 4 x 64:
-  // 106 at 8, 110 at 16).
+  // Head dimensions 64 and 128: a wave per (lane, KV head, split), splits of at least 4 pages, and at most so many
+  // waves to a launch.  The kernel (kvx_decode_small.hip) holds 4096 of them at 64 and 3072 at 128.  These
+  // numbers against 1024, 1536, 2048, 3072, 4096 and 6144 waves, ten batches of 1 to 32 sequences of 300 to
+  // 65 000 tokens each: at 8 x 4 x 64 the best of those for a format takes 1.00, 0.99, 0.98 and 0.97 of the time in
+  // the mean (int4, int8, e4m3, bf16), at 2 x 8 x 128 1024 waves take 0.94, 0.95 and 0.94 for int4, int8 and e4m3, whose
+  // launches end in a second round or in partial rows (32 sequences of 8192 tokens, int4: 37.7 us a layer in 52
+  // splits, 32.6 in 16; int8 38.3 in 29, 35.1 in 16), bf16 1.00.  The counts were set on an earlier kernel and stay:
+  // a row's bits depend on them, since weights are rounded against their split's running maximum.
   const bool sixteen = layout->head_dim == 64 || layout->format == KVX_FMT_INT4;
   const uint64_t slots = (sixteen ? 4096 : 2048) / (layout->format == KVX_FMT_BF16 ? 2 : 1);
   for (uint32_t first = 0; first < n_lanes; first += KVX_LANES_PER_LAUNCH) {
@@ -397,12 +397,11 @@ int kvx_decode_plan_for(const kvx_layout *layout, const uint32_t *committed, uin
 static void verify_plan_of_launch(const uint32_t *committed, uint32_t n_lanes, uint32_t rows,
                                   uint32_t kv_heads, uint32_t query_heads, uint32_t format,
                                   uint32_t *split_counts) {
-  // The verify kernels keep 32 fused rows (16 when there are no more; all of 33 .. 48
-  // on int4 pages) per wave and run one wave per SIMD, so a launch is (sum of splits) x KV heads x row blocks
-  // waves: the plan is the longest split length that still gives every SIMD of
-  // 256 CUs x 4 a wave, but no more waves than SIMDs, so that no second round of
-  // waves starts on a nearly empty GPU; splits shorter than 8 pages cost more in
-  // set-up and partial rows than they win.
+  // A launch is counted as (sum of splits) x KV heads x row blocks on the 256 CUs x 4 SIMDs: a block is a
+  // wave of 32 fused rows (16 when there are no more; all of 33 .. 48 on int4 pages), or a share of a
+  // workgroup that verify_row_blocks has.  The plan is the longest split length that still gives every SIMD a
+  // block, but no more blocks than SIMDs, so that no second round starts on a nearly empty GPU;
+  // splits shorter than 8 pages cost more in set-up and partial rows than they win.
   const uint32_t fused = rows * (query_heads / kv_heads);
   const uint32_t blocks = kvx::verify_row_blocks(format, fused);
   // The int4 kernel for lanes of more than 32 fused rows in blocks of 32 is built for two

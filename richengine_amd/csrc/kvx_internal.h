@@ -206,10 +206,14 @@ inline uint32_t prefill_group_width(uint32_t format, uint32_t head_dim, uint32_t
 inline bool prefill_group_splits_alike(uint32_t width, uint32_t committed) {
   return width == 4 ? committed % KVX_PAGE_TOKENS == 0 : prefill_tiles_pair(committed);
 }
-// Waves (row blocks) per (lane, split, KV head) of a verify launch.
+// Row blocks per (lane, split, KV head) of a verify launch, of which a round of the GPU holds 1024
+// (one to a SIMD).
 inline uint32_t verify_row_blocks(uint32_t format, uint32_t fused_rows) {
-  // bf16, fp8, int8 pages: 65 .. 128 fused rows run as four waves that share their pages
-  // (bf16 up to 96 rows: as two waves of 48).
+  // bf16, fp8 and int8 pages, more than 32 fused rows: a workgroup per (lane, split, KV head), two of them to a CU
+  // up to 64 rows (bf16: 96), one above, so that a round is 512 or 256 of them.  With 0.5, 0.67, 0.8, 1.25, 1.5 and
+  // 2 times the splits that follow, 36 to 96 rows over eight batches of 1 to 32 lanes took 1.16, 1.14, 1.07,
+  // 1.17, 1.13 and 1.17 times as long (int8, 48 rows; 96 rows 1.41, 1.31, 1.11, 1.25, 1.18, 1.10; e4m3 the same),
+  // on bf16 pages 1.11, 1.08, 1.04, 1.18, 1.16, 1.24 and 1.03, 1.03, 1.00, 1.16, 1.15, 1.28.
   if (format == KVX_FMT_BF16 && fused_rows > 64 && fused_rows <= 96) return 2;
   if (format != KVX_FMT_INT4 && fused_rows > 64 && fused_rows <= 128) return 4;
   const uint32_t rows = verify_block_rows(format, fused_rows);

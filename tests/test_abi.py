@@ -294,8 +294,8 @@ def test_decode_and_verify_plans_size_the_launch_for_the_gpu():
     with pytest.raises(kvx.KvxError):
         kvx.prefill_plan(16384, 256, 4, 6)
     assert kvx.verify_plan([65536] * 4, 16, H, QH) == [21] * 4          # three waves of 32 fused rows
-    assert kvx.verify_plan([65536] * 4, 16, H, QH, kvx.BF16) == [32] * 4  # two waves of 48 rows that share their pages
-    assert kvx.verify_plan([65536] * 4, 16, H, QH, kvx.INT8) == [16] * 4  # four waves that share their pages
+    assert kvx.verify_plan([65536] * 4, 16, H, QH, kvx.BF16) == [32] * 4  # two workgroups to a CU: 512 in a round
+    assert kvx.verify_plan([65536] * 4, 16, H, QH, kvx.INT8) == [16] * 4  # one workgroup to a CU: 256 in a round
     with pytest.raises(kvx.KvxError):
         kvx.verify_plan([10], 8, 4, 6)
 
@@ -430,7 +430,7 @@ def test_prefill_groups_of_tiles_rule():
 
 
 def test_prefill_plan_by_layout():
-    """kvx_prefill_plan_for: head dimension 256 is kvx_prefill_plan_batch; 64 and 128 take the fewest
+    """kvx_prefill_plan_for: head dimension 256 is kvx_prefill_plan_batch (tests/test_prefill_plan.py); 64 and 128 take the fewest
     splits that make 4096 workgroups (groups of tiles counted as the kernels form them), none
     shorter than 4 pages."""
     import ctypes as C
