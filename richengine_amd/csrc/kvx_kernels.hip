@@ -2230,6 +2230,25 @@ uint64_t slot_bytes(uint64_t rows, uint32_t head_dim) {
 }
 }  // namespace
 
+namespace {
+// Whether the rows over a shared prefix are stacked and masked first, by a launch of 4.9 us, for the kernels that
+// take a lane's rows side by side: int4 prefixes of up to 16 fused rows (the decode kernel), int8 and bf16 ones of up
+// to 32 (attend_wide_kernel, single waves).  Every other prefix's rows are read where they lie; on int8 and bf16
+// pages that is verify_lane_kernel, a workgroup per (split, KV head), of which 512 are on the GPU at once.  Up to there
+// it takes 0.68 to 0.96 of the waves' time and their launch's (1 to 5 sequences over 1024 to 65 536 tokens,
+// 1 x 16 to 16 x 8 heads).  More of them run in rounds, with most of the rows of each empty: int8, 131 072
+// tokens, 6 x 6, 12 rows 103 us as waves, 130 as workgroups; 40 960 at 12 x 1, 4 rows 77 / 84; bf16, 131 072 at 5 x 3, 12
+// rows 153 / 170, but from 768 on 88 / 86 (40 960 at 8 x 4, 4 rows).  int8 waves of 17 to 32 rows are one to a SIMD, and
+// win where a split is long: 24 rows at 6 x 6, 10 pages a split 77 / 71 us, 32 pages 121 / 133.
+bool prefix_rows_stacked(uint32_t format, uint32_t kv_heads, uint32_t fused_rows, uint64_t tokens, uint32_t splits) {
+  if (format == KVX_FMT_INT4) return fused_rows <= 16;
+  const uint64_t pages = (tokens + kPage - 1) / kPage, per = (pages + splits - 1) / splits;
+  const uint64_t workgroups = (pages + per - 1) / per * kv_heads;
+  if (fused_rows > 32 || workgroups <= 512) return false;
+  return format == KVX_FMT_BF16 ? workgroups <= 768 : fused_rows <= 16 || per > 12;
+}
+}  // namespace
+
 uint64_t kvx_attend_shared_workspace_bytes(const kvx_verify_params *lanes, uint32_t n_lanes,
                                            uint32_t prefix_splits, uint32_t query_heads,
                                            const kvx_layout *layout) {
@@ -2316,9 +2335,7 @@ int kv_attend_decode_shared(const kvx_storage *s, uint32_t layer, uint32_t query
   const hipStream_t st = static_cast<hipStream_t>(stream);
   Epilogue partials{nullptr, nullptr, true}, prefix_partials = partials;
   const uint64_t *prefix_table[1] = {page_tables[0]};
-  // int4 prefixes of up to 16 fused rows run on the decode kernel, which takes a lane's rows side by side and
-  // masks; every other kernel reads the rows where they lie (a launch of 4.9 us less).
-  const bool stacked = l.format == KVX_FMT_INT4 && n_lanes * G <= 16;
+  const bool stacked = prefix_rows_stacked(l.format, H, n_lanes * G, shared_tokens + n_lanes, prefix_splits);
   if (stacked) {
     hipLaunchKernelGGL(shared_stage_kernel, dim3(n_lanes, H), dim3(D), 0, st,
                        static_cast<const uint16_t *>(queries), staged, masks, n_lanes, H, G, row_stride);

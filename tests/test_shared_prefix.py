@@ -95,6 +95,10 @@ def group(request, monkeypatch):
     ((1, 16), 9, [31, 70, 0, 5, 6, 7, 8, 9], 2, 1),  # 128
     ((2, 8), 17, [1 + i for i in range(16)], 3, 32),  # 128, sixteen sequences
     ((3, 1), 8, [5, 45], 1, 4),                      # two fused rows
+    # more than 512 (split, KV head) pairs: up to 32 fused rows run as single waves on int8 and (to 768) bf16 pages
+    ((8, 1), 70, [5, 45], 70, 4),
+    ((16, 5), 100, [3, 40, 0, 64], 34, 2),           # 20 rows; int8: splits too short for it
+    ((16, 3), 700, [3, 40, 0, 64, 1, 2], 50, 1),     # 18 rows, 14 pages a split
 ], indirect=["group"])
 def test_shared_prefix_decode_matches_oracle(fmt, group, shared_pages, own_tokens, prefix_splits, row_stride):
     import torch
