@@ -10,9 +10,9 @@
 // Why this form: a wave per head over a staged copy of its values (attend_split_small_wave_kernel) took the
 // softmax of a page for the 4 or 8 columns a head has, and passed every value through LDS two or
 // four bytes at a time.  With the step's token stored here too, a layer at 8 x 4 x 64: 32 int8 sequences of 700 ..
-// 8192 tokens 62.3 -> 42 us, int4 63 -> 40, bf16 of half the length 48.6 -> 39, one of 500 int8 tokens 14.9 -> 12.0;
-// at 2 x 8 x 128, int4, 40 -> 32.6 and 18.4 -> 13.3, bf16 34 -> 33 and 15.1 -> 12.2.  Bound by the memory: 32 x 8192
-// int8 tokens of one layer take 49.9 us in this kernel, 5.7 TB/s, slabs of 2 KiB.
+// 8192 tokens 63.5 -> 40.9 us, int4 63.5 -> 39.0, bf16 of half the length 49.9 -> 36.4, one of 500 int8 tokens 15.0 ->
+// 12.1; at 2 x 8 x 128, int4, 40.1 -> 32.5 and 18.7 -> 13.2, bf16 31.5 -> 30.6 and 14.8 -> 12.0.  Bound by the memory:
+// 32 x 8192 int8 tokens, slabs of 2 KiB, take 60.9 us a layer with the merge, 4.7 TB/s.
 //
 // Lane geometry (t = lane & 15, g = lane >> 4): key operand row t of token block tb is token 8 (t / 4) + 4 tb +
 // t % 4, so that lane (t, g) holds column t's scores of tokens 8g .. 8g + 7; the value operands' k-slots are
@@ -286,7 +286,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES
     for (uint32_t i = 0; i < Page::kTiles; ++i) acc[c][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float row_max = -INFINITY, row_sum = 0.0f, weight_sum = 0.0f;
 
-  for (uint32_t at = begin; at < end; ++at) {
+  // A page of the split; kLast: its last, the only one that can hold slots past the visible tokens, behind which
+  // nothing is asked for.  (With the last page asked for once more, so that one copy of the code serves all, splits
+  // of two to four pages took a quarter to a half more of the memory: bf16, 8 x 4000 tokens at 8 x 8 x 128 in 64
+  // splits 51.7 us a layer, now 42.1; 11 sequences of 2938 .. 5876 at 3 x 16 x 128 under the plan 32.2, now 30.0;
+  // int8, 32 x 700 .. 8192 at 8 x 4 x 64 42.1, now 40.9.)
+  const auto attend = [&](uint32_t at, auto last) __attribute__((always_inline)) {
+    constexpr bool kLast = decltype(last)::value;
     f32x4 s[2];
 #pragma unroll
     for (uint32_t p = 0; p < P; ++p)
@@ -298,13 +304,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) s[tb][i] = p == 0 || own == p ? mine[i] : s[tb][i];
       }
-    // Past the end the last page is loaded again, so that every wait counts the same loads.
     const f32x4 page_ks[2] = {ks[0], ks[1]}, page_vs[2] = {vs[0], vs[1]};
     const Slab next = slab_at(upcoming);
-    fetch_keys(next);
-    upcoming = scalar_entry(entries, min(at + 2 - begin, last_slot));
+    if constexpr (!kLast) {
+      fetch_keys(next);
+      upcoming = scalar_entry(entries, min(at + 2 - begin, last_slot));
+    }
     const uint32_t first_token = at * kPage + 8 * g;
-    const bool whole = (at + 1) * kPage <= visible;
+    const bool whole = !kLast || (at + 1) * kPage <= visible;
     float score[8], local_max = -INFINITY;
 #pragma unroll
     for (uint32_t i = 0; i < 8; ++i) {
@@ -369,8 +376,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES
 #pragma unroll
     for (uint32_t c = 0; c < Page::kGroups; ++c)
       page.each_value(c, [&](uint32_t i, u32x4 v) { acc[c][i] = mfma16<FMT>(v, weights, acc[c][i]); });
-    fetch_values(next);
-  }
+    if constexpr (!kLast) fetch_values(next);
+  };
+  for (uint32_t at = begin; at + 1 < end; ++at) attend(at, std::false_type{});
+  attend(end - 1, std::true_type{});
 
   // The lanes of a column hold disjoint tokens.
   float sum = row_sum, bias = 0.0f;
@@ -434,12 +443,13 @@ int kvx_decode_small_launch(uint32_t format, const void *queries, float *partial
                             uint32_t max_splits, const FusedAppend *fused, hipStream_t stream) {
   const uint32_t D = a.head_dim, G = a.group, H = a.kv_heads;
   if (!kvx_decode_small_covers(format, D, G)) return KVX_EINVAL;
-  // Two heads to a wave for int4 pages of head dimension 64 (1 KiB of keys a head) once there are waves enough:
-  // 32 x 8192 tokens 60 -> 50 us, 16 x 100 .. 1500 (1000 waves of one head) 18.5 -> 18.0; 4 x 2000 (512 waves) 15.1 ->
-  // 16.6.  Other pages gain nothing or little (int8, 32 x 700 .. 8192 tokens 42.8 / 43.8 us, 32 x 8192 62 / 58).
+  // Two heads to a wave for int4 pages of head dimension 64 (1 KiB of keys a head) once there are more waves of one
+  // head than a round of 3072: 8 x 8192 tokens (3328 waves) 27.8 -> 25.4 us, 32 x 8192 60.4 -> 48.8, 32 x 700 .. 8192
+  // 42.9 -> 39.1; 24 x 2000 (3072) 20.2 -> 20.7, 8 x 2000 (1024) 14.4 -> 16.0.  Other pages gain nothing or little
+  // (int8, 32 x 700 .. 8192 tokens 42.8 / 43.8 us, 32 x 8192 62 / 58).
   uint64_t waves = 0;  // of one head each
   for (uint32_t i = 0; i < a.n_lanes; ++i) waves += uint64_t(a.lane[i].split_count) * H;
-  const uint32_t P = format == KVX_FMT_INT4 && D == 64 && H % 2 == 0 && 2 * G <= 16 && waves > 768 ? 2 : 1;
+  const uint32_t P = format == KVX_FMT_INT4 && D == 64 && H % 2 == 0 && 2 * G <= 16 && waves > 3072 ? 2 : 1;
   SmallToken token{};
   if (fused)
     token = {static_cast<const uint16_t *>(fused->keys), static_cast<const uint16_t *>(fused->values), fused->lane_stride,

@@ -372,11 +372,11 @@ int kvx_decode_plan_for(const kvx_layout *layout, const uint32_t *committed, uin
   // Head dimensions 64 and 128: a wave per (lane, KV head, split), splits of at least 4 pages, and at most so many
   // waves to a launch.  The kernel (kvx_decode_small.hip) holds 4096 of them at 64 and 3072 at 128.  These
   // numbers against 1024, 1536, 2048, 3072, 4096 and 6144 waves, ten batches of 1 to 32 sequences of 300 to
-  // 65 000 tokens each: at 8 x 4 x 64 the best of those for a format takes 1.00, 0.99, 0.98 and 0.97 of the time in
-  // the mean (int4, int8, e4m3, bf16), at 2 x 8 x 128 1024 waves take 0.94, 0.95 and 0.94 for int4, int8 and e4m3, whose
-  // launches end in a second round or in partial rows (32 sequences of 8192 tokens, int4: 37.7 us a layer in 52
-  // splits, 32.6 in 16; int8 38.3 in 29, 35.1 in 16), bf16 1.00.  The counts were set on an earlier kernel and stay:
-  // a row's bits depend on them, since weights are rounded against their split's running maximum.
+  // 65 000 tokens each: at 8 x 4 x 64 the best of those for a format takes 1.00 of the time in the mean, for bf16 0.98,
+  // at 2 x 8 x 128 1024 waves take 0.93, 0.95 and 0.95 for int4, int8 and e4m3, whose launches end in a second round
+  // or in partial rows (32 sequences of 8192 tokens, int4: 36.5 us a layer in 52 splits, 31.4 in 16; int8 36.6
+  // in 29, 33.8 in 16), bf16 1.00.  The counts were set on an earlier kernel and stay: a row's bits depend on
+  // them, since weights are rounded against their split's running maximum.
   const bool sixteen = layout->head_dim == 64 || layout->format == KVX_FMT_INT4;
   const uint64_t slots = (sixteen ? 4096 : 2048) / (layout->format == KVX_FMT_BF16 ? 2 : 1);
   for (uint32_t first = 0; first < n_lanes; first += KVX_LANES_PER_LAUNCH) {

@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("heads,group,dim", [(4, 6, 256), (3, 1, 256), (1, 16, 256),
-                                             (8, 4, 64), (2, 8, 128), (3, 5, 64), (5, 3, 128), (1, 16, 128), (6, 1, 64)])
+                                             (8, 4, 64), (2, 8, 128), (3, 5, 64), (5, 3, 128), (1, 16, 128), (6, 1, 64),
+                                             (16, 2, 64)])  # splits of a page: two int4 heads to a wave
 @pytest.mark.parametrize("fmt", A.FORMATS)
 @pytest.mark.parametrize("one_page_splits", [False, True])
 def test_token_stored_by_the_attention_kernel(heads, group, dim, fmt, one_page_splits):

@@ -13,8 +13,8 @@ import test_gpu_attention as A
 
 pytestmark = pytest.mark.gpu
 
-# (KV heads, group, head dimension), rows, lanes, splits; 32 lanes of (8, 4, 64): two int4 heads to a wave
-DECODE = [((8, 4, 64), 1, 2, 3), ((2, 8, 128), 1, 2, 5), ((3, 16, 64), 1, 1, 1), ((8, 4, 64), 1, 32, 4)]
+# (KV heads, group, head dimension), rows, lanes, splits; 3328 waves: two int4 heads to a wave
+DECODE = [((8, 4, 64), 1, 2, 3), ((2, 8, 128), 1, 2, 5), ((3, 16, 64), 1, 1, 1), ((8, 4, 64), 1, 32, 13)]
 VERIFY = [((4, 6, 256), 8, 2, 3), ((4, 6, 256), 16, 2, 5), ((2, 16, 256), 8, 1, 1)]
 COMMITTED = 420  # 421, 428 and 436 tokens: a last page partly filled
 
