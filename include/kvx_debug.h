@@ -29,9 +29,10 @@ uint32_t kvx_debug_prefill_tiles_together(const kvx_layout *layout, uint32_t que
                                           uint32_t committed_tokens, uint32_t rows, uint32_t splits);
 
 /* Fused query rows to a wave (16, 32 or 48) of a kv_attend_verify call of these lanes on int4 pages of head
-   dimension 256 (0: invalid arguments or other pages), so tests can tell which kernel a lane ran on. */
+   dimension 256 (0: invalid arguments or other pages), or with `single_tile` of the 8-row tile that a prefill
+   chunk leaves beside its pairs, so tests can tell which kernel a lane ran on. */
 uint32_t kvx_debug_int4_verify_rows(const kvx_layout *layout, uint32_t query_heads,
-                                    const kvx_verify_params *lanes, uint32_t n_lanes);
+                                    const kvx_verify_params *lanes, uint32_t n_lanes, uint32_t single_tile);
 
 /* Streams the pages of `page_table` (n_pages device entries of an int4, head dimension 256
    storage) with exactly the loads of the int4 decode kernel, two waves per SIMD, and nothing

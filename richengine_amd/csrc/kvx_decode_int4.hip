@@ -920,8 +920,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 using namespace kvx;
 
-// Fused rows to a wave, for lanes of more than 16.
-// 16 where the launch's waves then are all on the GPU at once (three to a SIMD) and no split is longer
+// Fused rows to a wave of the kernels with one register set of pages; 0 for those with two, whose waves have 16: lanes
+// of no more than 16, and the single tiles of a chunk, one of which it may leave beside its pairs.  Such a tile is one lane whose split is as long as the
+// chunk's history, of which as many waves as there are run side by side: 305 rows after 5760 tokens at 4 x 6 in one
+// split 513 us, with the tile as one wave of 48 rows a head 618; 328 rows of three sequences after 18 688 at
+// 3 x 5 1551 and 1885.
+// Other lanes: 16 where the launch's waves then are all on the GPU at once (three to a SIMD) and no split is longer
 // than 48 pages (32 with three to a SIMD: chains of 8 over 32 x 512 .. 16 384 tokens, 37 pages, 133 us, as 48 rows
 // 128): twice the waves of 32 rows, each through its page in half the time, and a GPU that
 // waves of 32 leave half empty is full (chains of 6 rows over 2 x 1000 tokens 20.8 -> 12.4 us, trees of 16
@@ -934,7 +938,8 @@ using namespace kvx;
 // bound by their instructions: 16 rows while that is a wave to a SIMD (512 rows after 512 tokens 74 -> 50 us,
 // two sequences of 300 after 4096 232 -> 171; with 1216 waves of 16 at 2 x 16 x 256 257 us, as 608 of 32 240).
 static uint32_t int4_blocks(uint32_t kv_heads, uint32_t fused_rows, const kvx_verify_params *lanes,
-                            uint32_t n_lanes, bool tiles) {
+                            uint32_t n_lanes, bool tiles, bool single_tiles) {
+  if (fused_rows <= 16 || single_tiles) return 0;
   uint64_t waves = 0;
   uint32_t longest = 0;
   const uint32_t launched = tiles ? n_lanes : std::min(n_lanes, kLanes);  // of the first launch
@@ -949,14 +954,16 @@ static uint32_t int4_blocks(uint32_t kv_heads, uint32_t fused_rows, const kvx_ve
 }
 
 extern "C" uint32_t kvx_debug_int4_verify_rows(const kvx_layout *layout, uint32_t query_heads,
-                                               const kvx_verify_params *lanes, uint32_t n_lanes) {
+                                               const kvx_verify_params *lanes, uint32_t n_lanes,
+                                               uint32_t single_tile) {
   if (!kvx_layout_valid(layout) || layout->format != KVX_FMT_INT4 || layout->head_dim != kD || !query_heads ||
       query_heads % layout->kv_heads || !lanes || !n_lanes)
     return 0;
   const uint32_t fused_rows = lanes[0].row_capacity * (query_heads / layout->kv_heads);
   for (uint32_t i = 0; i < n_lanes; ++i)
     if (!lanes[i].split_count) return 0;
-  return fused_rows <= 16 ? 16 : int4_blocks(layout->kv_heads, fused_rows, lanes, n_lanes, false);
+  const uint32_t rows = int4_blocks(layout->kv_heads, fused_rows, lanes, n_lanes, false, single_tile != 0);
+  return rows ? rows : 16;
 }
 
 // Runs paged attention (split kernel, then the merge of multi-split lanes) for
@@ -983,13 +990,13 @@ int kvx_attend_int4_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
   // The kernel appends the step's token itself only where one wave owns a
   // (sequence, KV head, split): one-row decode.
   if (fused && (fused_rows > 16 || lanes[0].row_capacity != 1)) return 1;
-  if (tile_rows && !fused && (many_tiles || fused_rows <= 16))
+  const uint32_t rows = int4_blocks(s->layout.kv_heads, fused_rows, lanes, n_lanes, tile_rows, many_tiles);
+  if (tile_rows && !rows)
     return launch_matrix_attention(decode_int4_tiles_kernel, "decode_int4_tiles_kernel", 16, 64, s,
                                    kv, query_heads, queries, output, page_tables, lanes, n_lanes,
                                    row_masks, row_stride, lane_stride, workspace, workspace_bytes,
                                    stream, nullptr, tile_rows, epilogue);
-  if (fused_rows > 16) {
-    const uint32_t rows = int4_blocks(s->layout.kv_heads, fused_rows, lanes, n_lanes, tile_rows);
+  if (rows) {
     if (rows == 48)
       return launch_matrix_attention(verify48_int4_kernel, "verify48_int4_kernel", 48, 64, s, kv,
                                      query_heads, queries, output, page_tables, lanes, n_lanes,

@@ -202,7 +202,7 @@ def _declare(L):
     L.kvx_debug_prefill_tiles_together.restype = u32
     L.kvx_debug_prefill_by_chunk.argtypes = [LP, u32, u32, u32, u32]
     L.kvx_debug_prefill_by_chunk.restype = u32
-    L.kvx_debug_int4_verify_rows.argtypes, L.kvx_debug_int4_verify_rows.restype = [LP, u32, vp, u32], u32
+    L.kvx_debug_int4_verify_rows.argtypes, L.kvx_debug_int4_verify_rows.restype = [LP, u32, vp, u32, u32], u32
     L.kvx_calibrate_stream.argtypes = [vp, u32, vp, u32, u32, u32, vp, vp]
     L.kvx_calibrate_stream_form.argtypes = [vp, u32, vp, u32, u32, u32, u32, u32, vp, vp]
     L.kvx_decode_plan.argtypes = [vp, u32, u32, u32, vp]

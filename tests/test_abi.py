@@ -484,3 +484,25 @@ def test_prefill_by_chunk_rule():
     assert by_chunk(8, 4, 64, kvx.INT4, 0, 1024, 32) == 0       # splits of a single page
     assert by_chunk(4, 6, 192, kvx.BF16, 0, 64, 1) == 0 and by_chunk(4, 0, 256, kvx.BF16, 0, 64, 1) == 0
     assert by_chunk(4, 6, 256, kvx.BF16, 0, 64, 33) == 0 and by_chunk(4, 6, 256, kvx.BF16, 0, 0, 1) == 0
+
+
+def test_int4_rows_to_a_wave_rule():
+    """kvx_debug_int4_verify_rows: 16 rows to a wave for lanes of no more and small launches of short splits, 32 or 48
+    for the others; the tile that a chunk leaves beside its pairs keeps waves of 16 however long its split is."""
+    import ctypes as C
+
+    def rows_to_a_wave(heads, group, committed, rows, splits, lanes=1, single_tile=0, fmt=kvx.INT4, dim=256):
+        layout = kvx.Layout(1, heads, dim, fmt, 0.0)
+        params = (kvx.VerifyParams * lanes)(*[kvx.VerifyParams(committed, (committed + rows + 31) // 32, kvx.KvLayer(),
+                                                               splits, splits, rows, rows, 0.0)] * lanes)
+        return kvx.lib().kvx_debug_int4_verify_rows(C.byref(layout), heads * group, params, lanes, single_tile)
+
+    assert rows_to_a_wave(4, 6, 5760, 1, 1) == 16 and rows_to_a_wave(4, 2, 5760, 8, 1) == 16
+    assert rows_to_a_wave(4, 6, 5760, 8, 1) == 48 and rows_to_a_wave(4, 6, 5760, 16, 1) == 32
+    assert rows_to_a_wave(4, 6, 5760, 8, 4) == 16           # 46 pages a split
+    assert rows_to_a_wave(4, 6, 5760, 16, 16, lanes=32) == 32
+    for heads, group in ((4, 6), (3, 5), (8, 4), (1, 16), (4, 3)):
+        for committed in (0, 1248, 5760, 65536):
+            assert rows_to_a_wave(heads, group, committed, 8, 1, single_tile=1) == 16
+    assert rows_to_a_wave(4, 6, 5760, 8, 1, fmt=kvx.INT8) == 0 and rows_to_a_wave(4, 6, 5760, 8, 1, dim=128) == 0
+    assert rows_to_a_wave(4, 6, 5760, 8, 0) == 0

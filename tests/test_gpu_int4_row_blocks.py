@@ -18,7 +18,7 @@ D = 256
 def rows_to_a_wave(heads, group, params):
     layout = kvx.Layout(2, heads, D, kvx.INT4, 0.0)
     lanes = (kvx.VerifyParams * len(params))(*params)
-    return kvx.lib().kvx_debug_int4_verify_rows(C.byref(layout), heads * group, lanes, len(params))
+    return kvx.lib().kvx_debug_int4_verify_rows(C.byref(layout), heads * group, lanes, len(params), 0)
 
 
 def verify(tw, tables, heads, group, q, params):
