@@ -562,6 +562,15 @@ __device__ __forceinline__ void attend_int4(const uint16_t *__restrict__ queries
     head = NB == 1 ? pair % args.kv_heads : pair / args.items;
     item = NB == 1 ? pair / args.kv_heads : pair - head * args.items;
     if (head >= args.kv_heads || item >= args.items) return;
+    // Tiles of a prefill, in launches of several rounds: those that see the most first, of every sequence in turn.
+    // (From the first tile on the longest waves began last: two chunks of 2048 rows after 512 tokens at 4 x 6 in one
+    // split 330 us a layer, so 297; three after 64 tokens 324 as single waves, whose order goes through the chunk once a
+    // head and block, so 264; four after 16 384 tokens 4126 as single waves, 3966 from the first tile on, 3897 so.)
+    if (NB == 2 && args.tile_lanes) {
+      const uint32_t splits = args.lane[0].split_count, rank = item / splits, per = args.tile_per_sequence;
+      const uint32_t sequences = args.tile_lanes / per;
+      item = (rank % sequences * per + per - 1 - rank / sequences) * splits + (item - rank * splits);
+    }
   }
   DecodeLane l;
   LaunchArgs a;
@@ -857,6 +866,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   attend_int4<2, 1, true, false, true>(queries, output, partials, statistics, a);
 }
 
+// Pairs of tiles in waves of 32 rows, a wave to a workgroup: launches that are on the GPU at once (2048 waves), which
+// single waves fill more evenly (four chunks of 448 rows after 64 tokens at 4 x 6, 1344 waves, 58.8 us a layer, as
+// workgroups of four 66.1; 400 rows 59.2 / 55.9, 640 rows 71.6 / 78.1), and those whose last wave is no more than
+// half full: where a wave that has less to do sits beside the others, its place is empty until the longest of them
+// ends (1126 rows of three sequences after 96 tokens at 3 x 5 148 / 157, 363 of sixteen after 64 at 4 x 3 79 / 83).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_int4_kernel(
+    const uint16_t *__restrict__ queries, uint16_t *__restrict__ output,
+    float *__restrict__ partials, float *__restrict__ statistics, DecodeArgs a) {
+  attend_int4<2, 1, true>(queries, output, partials, statistics, a);
+}
+
 // Single tiles of a chunked prefill, and pairs of no more than 16 fused rows: a wave to a workgroup with
 // two register sets of pages (as waves of verify_int4_kernel 256 rows after 8192 tokens in five splits
 // took 168 us instead of 133, one tile after 40 000 in sixteen 143 instead of 99).
@@ -996,6 +1016,13 @@ int kvx_attend_int4_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
                                    kv, query_heads, queries, output, page_tables, lanes, n_lanes,
                                    row_masks, row_stride, lane_stride, workspace, workspace_bytes,
                                    stream, nullptr, tile_rows, epilogue);
+  if (tile_rows && rows == 32) {
+    const uint64_t waves = uint64_t(n_lanes) * lanes[0].split_count * s->layout.kv_heads * ((fused_rows + 31) / 32);
+    if (waves <= 2048 || (fused_rows - 1) % 32 < 16)
+      return launch_matrix_attention(prefill_int4_kernel, "prefill_int4_kernel", 32, 64, s, kv, query_heads,
+                                     queries, output, page_tables, lanes, n_lanes, row_masks, row_stride,
+                                     lane_stride, workspace, workspace_bytes, stream, nullptr, tile_rows, epilogue);
+  }
   if (rows) {
     if (rows == 48)
       return launch_matrix_attention(verify48_int4_kernel, "verify48_int4_kernel", 48, 64, s, kv,

@@ -319,7 +319,7 @@ def test_hot_kernels_stay_out_of_scratch_memory():
         return report[names[0]]
 
     for fragment in ("decode_int4_kernelE", "decode_int4_quad_kernel", "decode_int4_tiles_kernel", "verify_int4_kernel",
-                     "verify32_int4_kernel", "verify48_int4_kernel",
+                     "verify32_int4_kernel", "verify48_int4_kernel", "prefill_int4_kernel",
                      "matrix_merge_kernelILj1E", "matrix_merge_kernelILj8E",   # one wave per row; ranged
                      "attend_wide_kernelILj1ELj1ELj2ELb0E",    # int8, one block, two waves per SIMD
                      "attend_wide_kernelILj4ELj1ELj2ELb0E",    # fp8
@@ -333,7 +333,7 @@ def test_hot_kernels_stay_out_of_scratch_memory():
         assert r["scratchsize"] == 0 and r["vgprs_spill"] == 0, (fragment, r)
     assert one("decode_int4_kernelE")["occupancy"] == 2 and one("decode_int4_quad_kernel")["occupancy"] == 2
     # two blocks over one page set: every accumulator in the first register file
-    assert one("verify32_int4_kernel")["agprs"] == 0
+    assert one("verify32_int4_kernel")["agprs"] == 0 and one("prefill_int4_kernel")["agprs"] == 0
     # waves of 16 rows: three to a SIMD
     assert one("verify_int4_kernel")["occupancy"] == 3
     # the workgroup-shared prefill kernels (int8, bf16, fp8 pages; two and three row blocks

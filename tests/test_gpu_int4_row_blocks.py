@@ -10,6 +10,7 @@ from oracle import kvoracle as ko
 from richengine_amd import kvx
 import gpulib as Gp
 import test_gpu_attention as A
+import test_gpu_prefill_batch as B
 
 pytestmark = pytest.mark.gpu
 D = 256
@@ -64,4 +65,22 @@ def test_a_lane_in_every_form(heads, group, rows, long_form, committed):
     alone = verify(tw, [long_td], heads, group, q, [halves])
     beside = verify(tw, [long_td, long_td], heads, group, np.repeat(q, 2, 0), [halves, long])
     assert np.array_equal(beside[0], alone[0])
+    tw.close()
+
+
+# pairs of tiles alone in waves of 16 rows, together in waves of 32: a wave to a workgroup up to 2048 of them and where
+# the last wave of a pair is half full (five blocks of 16), else four, those that see the most first; odd tiles beside the
+# pairs, histories that end anywhere, two splits
+@pytest.mark.parametrize("heads,group,committed,rows,splits,waves", [
+    (4, 6, (96, 0, 45, 1000), 264, 1, 768), (4, 6, (96, 0, 45, 100, 32, 7), 680, 1, 3024),
+    (2, 6, (64, 320, 0, 96, 32, 0), 515, 2, 2304), (3, 5, (96, 33, 7), 488, 1, 810), (8, 2, tuple(range(0, 320, 32)), 521, 1, 2640),
+    (1, 16, (31, 500, 0, 7, 64, 100, 200, 3, 90), 530, 1, 2376)])
+def test_pairs_of_tiles_of_several_sequences(monkeypatch, heads, group, committed, rows, splits, waves):
+    for name, value in zip(("H", "G", "D", "QH"), (heads, group, D, heads * group)):
+        monkeypatch.setattr(B, name, value)
+    n, pairs = len(committed), rows // 16 + (rows % 16 > 8)
+    assert n * pairs * heads * splits * group > 1024 and n * pairs * heads * splits * -(-group // 2) == waves
+    together, alone, tw = B.run_batch(ko.INT4, list(committed), [rows] * n, [splits] * n)
+    assert np.array_equal(together, alone)
+    assert (alone != 0x5A5A).any(axis=1).all()
     tw.close()
