@@ -698,8 +698,9 @@ int kv_attend_decode_static(const kvx_storage *storage, uint32_t layer, uint32_t
    elements apart) followed by kv_attend_decode over committed_tokens + 1 tokens.  The
    reference stores and attends in one call the same way (ops::PagedAttention::addVerify,
    runtime/ops/PagedAttention.cpp:467-544).  Same page bytes and same output as the two
-   calls; for groups of at most 16 query heads the wave that owns a sequence's last page stores
-   the token itself, which saves the append launch. */
+   calls; at head dimensions 64, 128 and 256 and groups of at most 16 query heads the wave that
+   owns a sequence's last page stores the token itself, which saves the append launch (unless the
+   call writes its output or partial rows into the chunk's memory). */
 int kv_append_attend_decode(const kvx_storage *storage, uint32_t layer, const void *chunk_keys,
                             const void *chunk_values, uint64_t chunk_lane_stride,
                             uint32_t chunk_stride, uint32_t query_heads, const void *queries,

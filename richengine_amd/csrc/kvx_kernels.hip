@@ -2493,6 +2493,20 @@ int kv_attend_decode_static(const kvx_storage *s, uint32_t layer, uint32_t query
 }
 
 namespace {
+// Whether a call writes (`to`, elements of two bytes; null: nothing) into the step's chunk rows of n_lanes lanes.
+// Where the attention kernel stores the tokens itself, it reads one lane's rows while another's output, hidden rows or
+// partial rows may be written; an append launch has read them all before.
+bool writes_chunk_rows(const void *to, uint64_t elements, const void *keys, const void *values, uint64_t lane_stride,
+                       uint32_t stride, uint32_t kv_heads, uint32_t head_dim, uint32_t n_lanes) {
+  const uint64_t lanes_before = uint64_t(n_lanes - 1) * lane_stride;
+  const auto meets = [&](const void *rows, uint64_t read) {
+    const uint64_t a = reinterpret_cast<uint64_t>(to), b = reinterpret_cast<uint64_t>(rows);
+    return a < b + 2 * (lanes_before + read) && b < a + 2 * elements;
+  };
+  return to && (meets(keys, uint64_t(kv_heads - 1) * stride * head_dim + head_dim) ||
+                meets(values, (uint64_t(kv_heads) * head_dim - 1) * stride + 1));
+}
+
 // kv_append_attend_decode and its form whose merge also writes the hidden rows (epilogue
 // given; `output` may then be null).
 int append_attend_decode(const kvx_storage *s, uint32_t layer, const void *chunk_keys,
@@ -2523,26 +2537,36 @@ int append_attend_decode(const kvx_storage *s, uint32_t layer, const void *chunk
     return rc;
   const uint32_t group = query_heads / s->layout.kv_heads;
   const uint64_t lane_stride = uint64_t(s->layout.kv_heads) * row_stride * group * s->layout.head_dim;
-  // int4 pages: the wave that owns a sequence's last page stores the token itself.
-  const int fused = kvx_attend_int4_launch(s, kv, query_heads, queries, output, page_tables, lanes,
-                                           n_lanes, nullptr, row_stride, lane_stride, workspace,
-                                           workspace_bytes, 0, static_cast<hipStream_t>(stream),
-                                           chunk_keys, chunk_values, chunk_lane_stride, chunk_stride, 0,
-                                           epilogue);
-  if (fused <= 0) return took(fused);
-  // bf16, e4m3 and int8 pages of head dimension 256 too.
-  const FusedAppend token{chunk_keys, chunk_values, chunk_lane_stride, chunk_stride};
-  const int wide = kvx_attend_wide_launch(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr,
-                                          row_stride, lane_stride, workspace, workspace_bytes, 0,
-                                          static_cast<hipStream_t>(stream), 0, epilogue, &token);
-  if (wide <= 0) return took(wide);
-  // The lanes of decode_small_kernel too.
-  if (kvx_decode_small_covers(s->layout.format, s->layout.head_dim, group)) {
-    took(1);
-    return attend_generic(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr, row_stride,
-                          workspace, static_cast<hipStream_t>(stream), epilogue, &token);
+  const auto onto_chunk = [&](const void *to, uint64_t elements) {
+    return writes_chunk_rows(to, elements, chunk_keys, chunk_values, chunk_lane_stride, chunk_stride,
+                             s->layout.kv_heads, s->layout.head_dim, n_lanes);
+  };
+  const bool apart =
+      !onto_chunk(output, n_lanes * lane_stride) &&
+      !onto_chunk(epilogue ? epilogue->hidden : nullptr, uint64_t(n_lanes) * query_heads * s->layout.head_dim) &&
+      !onto_chunk(workspace, kvx_attend_workspace_bytes(lanes, n_lanes, query_heads, &s->layout) / 2);
+  if (apart) {
+    // int4 pages: the wave that owns a sequence's last page stores the token itself.
+    const int fused = kvx_attend_int4_launch(s, kv, query_heads, queries, output, page_tables, lanes,
+                                             n_lanes, nullptr, row_stride, lane_stride, workspace,
+                                             workspace_bytes, 0, static_cast<hipStream_t>(stream),
+                                             chunk_keys, chunk_values, chunk_lane_stride, chunk_stride, 0,
+                                             epilogue);
+    if (fused <= 0) return took(fused);
+    // bf16, e4m3 and int8 pages of head dimension 256 too.
+    const FusedAppend token{chunk_keys, chunk_values, chunk_lane_stride, chunk_stride};
+    const int wide = kvx_attend_wide_launch(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr,
+                                            row_stride, lane_stride, workspace, workspace_bytes, 0,
+                                            static_cast<hipStream_t>(stream), 0, epilogue, &token);
+    if (wide <= 0) return took(wide);
+    // The lanes of decode_small_kernel too.
+    if (kvx_decode_small_covers(s->layout.format, s->layout.head_dim, group)) {
+      took(1);
+      return attend_generic(s, kv, query_heads, queries, output, page_tables, lanes, n_lanes, nullptr, row_stride,
+                            workspace, static_cast<hipStream_t>(stream), epilogue, &token);
+    }
   }
-  // Every other shape: the two entries one after the other.
+  // Every other call: the two entries one after the other.
   std::vector<kvx_chunk_params> chunks(n_lanes);
   for (uint32_t i = 0; i < n_lanes; ++i)
     chunks[i] = {lanes[i].committed_tokens, 1, chunk_stride, lanes[i].page_table_entries, {}};

@@ -72,3 +72,55 @@ def test_token_stored_by_the_attention_kernel(heads, group, dim, fmt, one_page_s
         assert np.array_equal(tw.dev.extent_read(e), after[e])
     assert torch.equal(one, two)
     tw.close()
+
+
+@pytest.mark.parametrize("heads,group,dim", [(4, 6, 256), (8, 4, 64), (2, 8, 128)])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+@pytest.mark.parametrize("written", ["output over keys", "output over values", "hidden", "workspace"])
+def test_a_call_that_writes_over_its_chunk_rows(heads, group, dim, fmt, written):
+    """What the step writes lies in the memory that its chunk rows came in: every row is stored first."""
+    lanes, n, splits = 40, 3, 1 if written.startswith("output") else 2
+    committed = [int(c) for c in np.random.default_rng(7).integers(64, 96, lanes)]
+    tw = Gp.Twin(fmt, heads, dim, 2, lanes * n)
+    ids, rng = tw.pages(lanes * n, 9), np.random.default_rng(8)
+    dts = [tw.tables(ids[n * i:n * i + n])[1] for i in range(lanes)]
+    rows = lambda *shape: rng.standard_normal(shape).astype(np.float32)
+    for lane, c in enumerate(committed):
+        ck, cv = T.chunk_buffers(rows(heads, c, dim), rows(heads, c, dim), 32 * n)
+        kvx.append(tw.dev, 1, Gp.dev(ck), Gp.dev(cv), [dts[lane]], [kvx.ChunkParams(0, c, 32 * n, n)], heads * 32 * n * dim)
+    chunks = [T.chunk_buffers(rows(heads, 1, dim), rows(heads, 1, dim), 32) for _ in range(lanes)]
+    keys, values = (Gp.dev(np.stack([c[i] for c in chunks])).flatten() for i in (0, 1))
+    q = Gp.dev(A.queries((lanes, heads, 1, group, dim), 63))
+    dp = [kvx.VerifyParams(c, n, kvx.KvLayer(), splits, splits, 1, 1, 0.0) for c in committed]
+    ws = torch.empty(kvx.attend_workspace_bytes(tw.dev, dp, heads * group), dtype=torch.uint8, device="cuda")
+    want = torch.zeros_like(q)
+    hidden_want = torch.zeros((lanes, 1, heads * group, dim), dtype=torch.int16, device="cuda")
+    torch.cuda.synchronize()
+    before = [tw.dev.extent_read(e).copy() for e in range(tw.extents)]
+    kvx.append(tw.dev, 1, keys, values, dts, [kvx.ChunkParams(c, 1, 32, n) for c in committed], heads * 32 * dim)
+    if written == "hidden":
+        kvx.attend_verify_hidden(tw.dev, 1, heads * group, q, want, dts, dp, None, 1, ws, None, hidden_want)
+    else:
+        kvx.attend_decode(tw.dev, 1, heads * group, q, want, dts, dp, 1, ws)
+    torch.cuda.synchronize()
+    after = [tw.dev.extent_read(e).copy() for e in range(tw.extents)]
+    for e in range(tw.extents):
+        tw.dev.extent_write(e, before[e])
+    args = (tw.dev, 1, keys, values, heads * 32 * dim, 32, heads * group, q)
+    if written == "hidden":
+        out, hidden = torch.zeros_like(q), keys[16:16 + hidden_want.numel()].view_as(hidden_want)
+        kvx.append_attend_decode_hidden(*args, out, dts, dp, 1, ws, None, hidden)
+    elif written == "workspace":
+        out, ws = torch.zeros_like(q), torch.cat([values, values.new_zeros(ws.numel())])
+        kvx.append_attend_decode(*args[:3], ws[:values.numel()], *args[4:], out, dts, dp, 1, ws.view(torch.uint8))
+    else:
+        over = keys if written == "output over keys" else values
+        out = over[:q.numel()].view_as(q)
+        kvx.append_attend_decode(*args, out, dts, dp, 1, ws)
+    torch.cuda.synchronize()
+    for e in range(tw.extents):
+        assert np.array_equal(tw.dev.extent_read(e), after[e])
+    assert torch.equal(out, want)
+    if written == "hidden":
+        assert torch.equal(hidden, hidden_want)
+    tw.close()
