@@ -491,7 +491,7 @@ def tree_verify(args):
         "value": round(lanes * nodes * args.steps / wall, 1), "unit": "draft tokens/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(wall * 1e3 / args.steps, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": {"int4": "int4 pages, bf16 MFMA", "int8": "int8 pages, fp16 MFMA",
+        "dtype": {"int4": "int4 pages, bf16 MFMA", "int8": "int8 pages, bf16 MFMA",
                   "bf16": "bf16 pages, bf16 MFMA"}[args.format] + ", fp32 accumulate", "data": "synthetic",
         "config": {"workload": "BASELINE configs[4]: speculative tree verify on " + args.format + " KV, batch 4, "
                                "contexts 65536, 16-node trees (branching <= 3), 16 layers: append 16 "
@@ -815,7 +815,7 @@ def shared_prefix(args):
                      "bytes_per_launch": physical,
                      "mfma_tflops": round(4 * D * QH * sum(c + 1 for c in committed) /
                                           (shared_ms * 1e-3) / 1e12, 1),
-                     "traffic": None, "kernel": "split kernels over the shared pages (stacked rows) and over the "
+                     "traffic": None, "kernel": "split kernels over the shared pages and over the "
                                                 "sequences' own pages + shared_merge_kernel",
                      "ms_per_launch": round(shared_ms, 4)},
         "unshared_ms": round(plain_ms, 4),
@@ -1044,7 +1044,7 @@ def chunked_prefill(args):
     torch.cuda.set_device(0)
     rng = np.random.default_rng(args.seed)
     fmt = {"bf16": kvx.BF16, "fp8": kvx.FP8, "int8": kvx.INT8, "int4": kvx.INT4}[args.format]
-    peak = 2500.0  # bf16 and fp16 MFMA (the one-byte formats multiply as fp16)
+    peak = 2500.0  # bf16 and fp16 MFMA (e4m3 multiplies as fp16)
     sequences, prefix, chunk = 4, 16384, args.prefill_chunk
     prefix_pages, chunk_pages = prefix // 32, chunk // 32
     total = prefix_pages + sequences * chunk_pages
@@ -1158,7 +1158,7 @@ def chunked_prefill(args):
         "steps": steps, "warmup": warmup, "ms_per_step": round(wall * 1e3 / steps, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": {"bf16": "bf16 pages, bf16 MFMA", "fp8": "fp8e4m3 pages, fp16 MFMA",
-                  "int8": "int8 pages, fp16 MFMA", "int4": "int4 pages, bf16 MFMA"}[args.format] +
+                  "int8": "int8 pages, bf16 MFMA", "int4": "int4 pages, bf16 MFMA"}[args.format] +
                  ", fp32 accumulate",
         "data": "synthetic",
         "config": {"workload": "BASELINE configs[3]: chunked prefill with a shared prefix, batch 4, "
@@ -1393,7 +1393,7 @@ def decode_layout(args):
         "pct_hbm_peak": round(100 * value / HBM_PEAK_GBS, 2),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "attend_split_small_wave_kernel (a wave per sequence, KV head and split)",
+                     "kernel": "decode_small_kernel (a wave per sequence, split and one or two KV heads)",
                      "bytes_per_launch": kv_bytes, "ms_per_launch": round(split_s * 1e3, 4),
                      "reduce_ms_per_launch": round(merge_s * 1e3, 4)},
         "cpu_baseline": None,

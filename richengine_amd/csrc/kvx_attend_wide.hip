@@ -1021,9 +1021,9 @@ int kvx_attend_wide_launch(const kvx_storage *s, kvx_kv_layer kv, uint32_t query
     return KVX_GROUP_FORMATS(2);
   }
   // Verify lanes of more than 32 fused rows, which hold 128 at most, and the rows of sequences over a prefix they
-  // share: waves that multiply beside waves that stage.  (Few workgroups are as fast, 16 lanes of 1200 tokens at
-  // 108 rows 30.1 / 28.8 us, so bf16 lanes of more than 96 rows take four waves of 32 rows here too; over 40 lanes
-  // of 1875 .. 3750 tokens, 112 rows, in the four waves of group_wide_kernel 99 us, in these 102.)
+  // share: waves that multiply beside waves that stage.  Not bf16 lanes of more than 96 rows, which keep the four
+  // waves of group_wide_kernel: 40 lanes of 1875 .. 3750 tokens, 112 rows, 99 us in those, 102 in these; few
+  // workgroups are as fast (16 lanes of 1200 tokens, 108 rows, 28.8 / 30.1 us).
   const bool shared_prefix = epilogue && epilogue->row_pitch;
   if (!tile_rows && !many_tiles && (M > 32 || shared_prefix) && M <= 32u * kGroupWaves) {
     if (format != KVX_FMT_BF16 || M <= 96 || shared_prefix)

@@ -10,9 +10,9 @@
 // Why this form: a wave per head over a staged copy of its values (attend_split_small_wave_kernel) took the
 // softmax of a page for the 4 or 8 columns a head has, and passed every value through LDS two or
 // four bytes at a time.  With the step's token stored here too, a layer at 8 x 4 x 64: 32 int8 sequences of 700 ..
-// 8192 tokens 63.5 -> 40.9 us, int4 63.5 -> 39.0, bf16 of half the length 49.9 -> 36.4, one of 500 int8 tokens 15.0 ->
-// 12.1; at 2 x 8 x 128, int4, 40.1 -> 32.5 and 18.7 -> 13.2, bf16 31.5 -> 30.6 and 14.8 -> 12.0.  Bound by the memory:
-// 32 x 8192 int8 tokens, slabs of 2 KiB, take 60.9 us a layer with the merge, 4.7 TB/s.
+// 8192 tokens 62.0 -> 40.0 us, int4 63.0 -> 37.4, bf16 of half the length 49.6 -> 37.1, one of 500 int8 tokens 15.5 ->
+// 12.9; at 2 x 8 x 128, int4, 40.0 -> 31.3 and 18.8 -> 13.8, bf16 33.4 -> 29.9 and 15.3 -> 12.8.  Bound by the memory:
+// 32 x 8192 int8 tokens, slabs of 2 KiB, take 49.3 us in this kernel, 5.8 TB/s, and 61.7 a layer with the merge.
 //
 // Lane geometry (t = lane & 15, g = lane >> 4): key operand row t of token block tb is token 8 (t / 4) + 4 tb +
 // t % 4, so that lane (t, g) holds column t's scores of tokens 8g .. 8g + 7; the value operands' k-slots are

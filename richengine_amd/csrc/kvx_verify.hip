@@ -1,6 +1,6 @@
-// Verify lanes of 33 to 128 fused query rows on bf16, e4m3 and int8 pages for gfx950, and the shared
-// prefix of such pages: the rows of one (lane, split, KV head) share every page through LDS (head
-// dimension 256).
+// Verify lanes of 33 to 128 fused query rows on e4m3 and int8 pages and of 33 to 96 on bf16 pages for
+// gfx950 (more on bf16 are group_wide_kernel's), and the shared prefix, up to 128 rows, of bf16 and int8
+// pages: the rows of one (lane, split, KV head) share every page through LDS (head dimension 256).
 //
 // A workgroup is R waves of 32 fused rows each and S waves that bring the pages: a page comes in
 // once, is expanded once into 16-bit MFMA operands in LDS (two copies, a barrier a page) and is

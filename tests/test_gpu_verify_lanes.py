@@ -1,6 +1,7 @@
-"""Verify lanes of 33 to 128 fused rows on bf16, int8 and e4m3 pages run as waves of 32 rows beside waves
-that stage the pages (kvx_verify.hip): the number of row waves, a last wave partly filled, live rows below
-the capacity, one split (rows written directly) and several, splits of one page."""
+"""Verify lanes of 33 to 128 fused rows on int8 and e4m3 pages, and of 33 to 96 on bf16 pages, run as waves of 32
+rows beside waves that stage the pages (kvx_verify.hip): the number of row waves, a last wave partly filled, live
+rows below the capacity, one split (rows written directly) and several, splits of one page.  bf16 lanes of 98 and
+128 rows run on group_wide_kernel (kvx_attend_wide.hip); tests/test_shared_prefix.py has the other form's."""
 import numpy as np
 import pytest
 import torch
