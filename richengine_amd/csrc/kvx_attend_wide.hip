@@ -203,9 +203,9 @@ __device__ __forceinline__ void append_wide_token(const DecodeArgs &a, const Dec
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) store_global<uint16_t>(data + ((4 * lane + i) * kPage + slot) * 2, row[1][i]);
     } else {
-      float maximum = 0.0f;
+      float maximum = fabsf(bf16_to_f32(row[tensor][0]));  // (not from 0: a row of nothing but NaN has no maximum)
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) maximum = fmaxf(maximum, fabsf(bf16_to_f32(row[tensor][i])));
+      for (uint32_t i = 1; i < 4; ++i) maximum = fmaxf(maximum, fabsf(bf16_to_f32(row[tensor][i])));
       for (int offset = 32; offset; offset >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, offset));
       constexpr float kMost = FMT == KVX_FMT_INT8 ? 127.0f : 448.0f;
       uint32_t packed = 0;

@@ -63,9 +63,9 @@ __device__ __forceinline__ void append_small_token(const SmallToken &a, const At
 #pragma unroll
       for (uint32_t i = 0; i < E; ++i) store_global<uint16_t>(data + 2 * at(E * lane + i), row[tensor][i]);
     } else {
-      float maximum = 0.0f;
+      float maximum = fabsf(bf16_to_f32(row[tensor][0]));  // (not from 0: a row of nothing but NaN has no maximum)
 #pragma unroll
-      for (uint32_t i = 0; i < E; ++i) maximum = fmaxf(maximum, fabsf(bf16_to_f32(row[tensor][i])));
+      for (uint32_t i = 1; i < E; ++i) maximum = fmaxf(maximum, fabsf(bf16_to_f32(row[tensor][i])));
       for (int offset = 32; offset; offset >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, offset));
       constexpr float kMost = FMT == KVX_FMT_INT4 ? 7.0f : FMT == KVX_FMT_INT8 ? 127.0f : 448.0f;
       constexpr int kLimit = FMT == KVX_FMT_INT4 ? 7 : 127;

@@ -124,3 +124,45 @@ def test_a_call_that_writes_over_its_chunk_rows(heads, group, dim, fmt, written)
     if written == "hidden":
         assert torch.equal(hidden, hidden_want)
     tw.close()
+
+
+@pytest.mark.parametrize("heads,group,dim", [(4, 6, 256), (8, 4, 64), (2, 8, 128)])
+@pytest.mark.parametrize("fmt", A.FORMATS)
+def test_tokens_that_are_no_numbers(heads, group, dim, fmt):
+    """Rows of nothing but NaN, with one, with infinities of either sign, with both: the bytes of kv_append."""
+    n, committed = 2, [40, 41, 42, 43, 44, 45, 46, 47]
+    lanes, rng = len(committed), np.random.default_rng(9)
+    tw = Gp.Twin(fmt, heads, dim, 2, lanes * n)
+    ids = tw.pages(lanes * n, 9)
+    dts = [tw.tables(ids[n * i:n * i + n])[1] for i in range(lanes)]
+    for lane, c in enumerate(committed):
+        ck, cv = T.chunk_buffers(*(rng.standard_normal((heads, c, dim)).astype(np.float32) for _ in range(2)), 32 * n)
+        kvx.append(tw.dev, 1, Gp.dev(ck), Gp.dev(cv), [dts[lane]], [kvx.ChunkParams(0, c, 32 * n, n)], heads * 32 * n * dim)
+    rows = rng.standard_normal((2, lanes, heads, 1, dim)).astype(np.float32)
+    rows[:, 0] = np.nan
+    rows[0, 1], rows[1, 2] = np.nan, np.nan
+    rows[:, 3, ..., 5] = np.nan
+    rows[:, 4, ..., 5] = np.inf
+    rows[:, 5, ..., dim - 1] = -np.inf
+    rows[:, 6, ..., 1:] = np.nan
+    rows[:, 7, ..., ::2], rows[:, 7, ..., 1] = np.nan, np.inf
+    chunks = [T.chunk_buffers(rows[0, i], rows[1, i], 32) for i in range(lanes)]
+    keys, values = (Gp.dev(np.stack([c[i] for c in chunks])).flatten() for i in (0, 1))
+    q = Gp.dev(A.queries((lanes, heads, 1, group, dim), 63))
+    dp = [kvx.VerifyParams(c, n, kvx.KvLayer(), 2, 2, 1, 1, 0.0) for c in committed]
+    ws = torch.empty(kvx.attend_workspace_bytes(tw.dev, dp, heads * group), dtype=torch.uint8, device="cuda")
+    two, one = torch.zeros_like(q), torch.zeros_like(q)
+    torch.cuda.synchronize()
+    before = [tw.dev.extent_read(e).copy() for e in range(tw.extents)]
+    kvx.append(tw.dev, 1, keys, values, dts, [kvx.ChunkParams(c, 1, 32, n) for c in committed], heads * 32 * dim)
+    kvx.attend_decode(tw.dev, 1, heads * group, q, two, dts, dp, 1, ws)
+    torch.cuda.synchronize()
+    after = [tw.dev.extent_read(e).copy() for e in range(tw.extents)]
+    for e in range(tw.extents):
+        tw.dev.extent_write(e, before[e])
+    kvx.append_attend_decode(tw.dev, 1, keys, values, heads * 32 * dim, 32, heads * group, q, one, dts, dp, 1, ws)
+    torch.cuda.synchronize()
+    for e in range(tw.extents):
+        assert np.array_equal(tw.dev.extent_read(e), after[e])
+    assert torch.equal(one, two)
+    tw.close()
